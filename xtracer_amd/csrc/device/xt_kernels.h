@@ -32,10 +32,12 @@ enum {
     CNT_WORDS = 8
 };
 #define XT_TRACE_SEGMENTS 8  // XCDs of an MI355X: one trace-queue segment each
+#define XT_CURSOR_STRIDE 32
 struct Counters {
     uint32_t n[CNT_WORDS];
     uint32_t seg[XT_TRACE_SEGMENTS];  // work cursors of the trace queue's segments (reset with CNT_CURSOR)
     unsigned long long queries, retests, steps_exceeded, trace_fail;
+    uint32_t xcd[XT_TRACE_SEGMENTS * XT_CURSOR_STRIDE];  // work cursors, one L2 line each (reset with CNT_CURSOR)
 };
 
 struct Queue {
@@ -105,7 +107,7 @@ __device__ __forceinline__ bool slot_pixel(const JobDev &j, uint32_t q, uint32_t
 static __global__ void k_reset(Counters *c, uint32_t mask) {
     const uint32_t i = threadIdx.x;
     if (i < CNT_WORDS && (mask >> i) & 1u) c->n[i] = 0;
-    if (i < XT_TRACE_SEGMENTS && (mask >> CNT_CURSOR) & 1u) c->seg[i] = 0;
+    if (i < XT_TRACE_SEGMENTS && (mask >> CNT_CURSOR) & 1u) c->seg[i] = c->xcd[i * XT_CURSOR_STRIDE] = 0;
     if (i == 0 && (mask >> 31) & 1u) {
         c->queries = 0;
         c->retests = 0;
@@ -119,7 +121,7 @@ static __global__ void k_reset_lanes(Counters *c, uint32_t mask) {
     Counters *b = c + blockIdx.x;
     const uint32_t i = threadIdx.x;
     if (i < CNT_WORDS && (mask >> i) & 1u) b->n[i] = 0;
-    if (i < XT_TRACE_SEGMENTS && (mask >> CNT_CURSOR) & 1u) b->seg[i] = 0;
+    if (i < XT_TRACE_SEGMENTS && (mask >> CNT_CURSOR) & 1u) b->seg[i] = b->xcd[i * XT_CURSOR_STRIDE] = 0;
     if (i == 0 && (mask >> 31) & 1u) {
         b->queries = 0;
         b->retests = 0;
@@ -427,21 +429,17 @@ __device__ __forceinline__ uint32_t seg_begin(uint32_t n, uint32_t s, uint32_t n
     return (uint32_t)((uint64_t)n * s / nseg) / G * G;
 }
 
-// Persistent trace: each wave takes XT_TRACE_CHUNK x 64 consecutive rays at
-// a time from a device cursor (one atomic per chunk) until the queue is
-// drained, so waves that drew short traversals pick up more work instead of
-// idling. With nseg = 8 the queue is cut into 8 contiguous segments with a
+// Persistent trace over the octree (parity mode): each wave takes 64
+// consecutive rays at a time from a device cursor (one atomic) until the queue
+// is drained. With nseg = 8 the queue is cut into 8 contiguous segments with a
 // cursor each; workgroups are dispatched to the 8 XCDs round-robin, so the
 // waves of XCD (block % 8) drain that segment first and then help with the
-// others. Rays next to each other in a queue come from neighbouring pixels,
-// so each XCD's L2 then holds the nodes and leaves of one part of the image
-// rather than of all of it.
-template <int ACCEL, int STACK, int BS>
-static __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(6))) void k_trace(const SceneView S, const Queue in, const uint32_t *in_count,
-                                                     float4 *hit, uint32_t *retest_list, uint4 *recheck_list,
-                                                     Counters *cnt, uint32_t nseg) {
-    __shared__ uint2 kstk[ACCEL == XT_ACCEL_KDTREE ? (STACK + 1) * BS : 1];
-    __shared__ uint32_t ostk[ACCEL == XT_ACCEL_OCTREE ? XT_OCT_STACK * BS : 1];
+// others.
+static __global__ __launch_bounds__(XT_OCT_BLOCK) void k_trace_oct(const SceneView S, const Queue in,
+                                                            const uint32_t *in_count, float4 *hit,
+                                                            uint32_t *retest_list, uint4 *recheck_list, Counters *cnt,
+                                                            uint32_t nseg) {
+    __shared__ uint32_t ostk[XT_OCT_STACK * XT_OCT_BLOCK];
     const uint32_t n = *in_count;
     if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&cnt->queries, (unsigned long long)n);
     const uint32_t lane = lane_id();
@@ -490,8 +488,7 @@ static __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(6))) 
             for (uint32_t k = 0; k < S.n_planes; ++k)
                 if (XT_PLANE_BASE + k != r.origin) plane32(r.o, r.d, tst.tsmall, S.planes[k], XT_PLANE_BASE + k, tst.best);
             bool ok;
-            if (ACCEL == XT_ACCEL_KDTREE) ok = walk_kd<STACK>(S, tst, r.o, r.d, kstk + threadIdx.x, BS, 1e-6f);
-            else ok = walk_oct(S, tst, r.o, r.d, ostk + threadIdx.x, BS, 1e-6f);
+            ok = walk_oct(S, tst, r.o, r.d, ostk + threadIdx.x, XT_OCT_BLOCK, 1e-6f);
             Best &bb = tst.best;
             // a deferred candidate matters only up to the closest hit (a miss
             // has t = INF, so compare only when something was deferred)
@@ -518,6 +515,8 @@ static __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(6))) 
         if (rc) recheck_list[cslot] = make_uint4(i, c0, c1, XT_NONE);
     }
 }
+
+#include "xt_trace_kd.h"
 
 __device__ __forceinline__ uint32_t object_of(const SceneView &S, uint32_t p) {
     return p >= XT_PLANE_BASE ? S.planes[p - XT_PLANE_BASE].object : __float_as_uint(S.prims[3 * p + 1].w);

@@ -86,54 +86,6 @@ struct Tester32 {
         const float4 a = S.prims[3 * prim], b = S.prims[3 * prim + 1], c = S.prims[3 * prim + 2];
         test_rec(prim, a, b, c);
     }
-    // kd leaf references [k, k + n): each record's three loads go out
-    // together, and the next record's while this one is tested (the empty
-    // asm keeps the compiler from sinking loads into the branches that use
-    // them, which would cost extra memory round trips)
-    __device__ __forceinline__ void test_leaf_range(uint32_t k, uint32_t n) {
-        if (n == 0) return;
-        if (S.kd_indexed) {
-            test_leaf_indexed(k, n);
-            return;
-        }
-        float4 a = S.kd_leaf[3 * k], b = S.kd_leaf[3 * k + 1], c = S.kd_leaf[3 * k + 2];
-        for (uint32_t j = 1; j <= n; ++j) {
-            float4 na = a, nb = b, nc = c;
-            if (j < n) {
-                const uint32_t q = 3 * (k + j);
-                na = S.kd_leaf[q];
-                nb = S.kd_leaf[q + 1];
-                nc = S.kd_leaf[q + 2];
-            }
-            asm volatile("" ::"v"(c.x), "v"(c.y), "v"(c.z), "v"(c.w));
-            test_rec(__float_as_uint(b.w), a, b, c);
-            a = na;
-            b = nb;
-            c = nc;
-        }
-    }
-    // the same through the reference list: one soup record per reference,
-    // the next reference's record loaded while this one is tested
-    __device__ __forceinline__ void test_leaf_indexed(uint32_t k, uint32_t n) {
-        uint32_t p = S.kd_refs[k];
-        float4 a = S.prims[3 * p], b = S.prims[3 * p + 1], c = S.prims[3 * p + 2];
-        for (uint32_t j = 1; j <= n; ++j) {
-            float4 na = a, nb = b, nc = c;
-            uint32_t np = p;
-            if (j < n) {
-                np = S.kd_refs[k + j];
-                na = S.prims[3 * np];
-                nb = S.prims[3 * np + 1];
-                nc = S.prims[3 * np + 2];
-            }
-            asm volatile("" ::"v"(c.x), "v"(c.y), "v"(c.z), "v"(c.w));
-            test_rec(p, a, b, c);
-            a = na;
-            b = nb;
-            c = nc;
-            p = np;
-        }
-    }
 };
 
 struct Tester64 {

@@ -133,11 +133,11 @@ extern "C" {
 // a device address: xt_dev_create looks its address up per device.
 struct StaticTraceScratch {
     Counters cnt;
-    uint32_t pad[64 - sizeof(Counters) / 4];
+    uint32_t pad[512 - sizeof(Counters) / 4];
     uint4 recheck[XT_TRACE_STATIC_MAX_RAYS];
     uint32_t retest[XT_TRACE_STATIC_MAX_RAYS];
 };
-static_assert(sizeof(Counters) % 4 == 0 && sizeof(Counters) < 256, "scratch header");
+static_assert(sizeof(Counters) % 4 == 0 && sizeof(Counters) < 2048, "scratch header");
 __device__ __align__(256) StaticTraceScratch scratch;
 
 int xt_dev_create(xt_dev **out, int hip_device, uint64_t hbm_budget_bytes) {
@@ -441,7 +441,7 @@ static void launch_kd_trace_sb(unsigned per_cu, int n_cu, size_t cap, hipStream_
     if (per_cu == 0) {
         if (resident == 0) {
             int nb = 0;
-            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_trace<XT_ACCEL_KDTREE, STACK, BS>, BS, 0) !=
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_trace_kd<STACK, BS>, BS, 0) !=
                     hipSuccess ||
                 nb < 1)
                 nb = 1;
@@ -451,7 +451,7 @@ static void launch_kd_trace_sb(unsigned per_cu, int n_cu, size_t cap, hipStream_
     }
     const size_t need = (cap + BS - 1) / BS;
     const unsigned g = (unsigned)std::max<size_t>(1, std::min<size_t>(need, (size_t)n_cu * per_cu));
-    hipLaunchKernelGGL((k_trace<XT_ACCEL_KDTREE, STACK, BS>), dim3(g), dim3(BS), 0, st, v, q, count, hit, retest, recheck,
+    hipLaunchKernelGGL((k_trace_kd<STACK, BS>), dim3(g), dim3(BS), 0, st, v, q, count, hit, retest, recheck,
                        cnt, nseg);
 }
 
@@ -486,7 +486,7 @@ int xt_launch_trace_bufs(xt_dev *d, const DevScene &ds, int accel, const TraceBu
     if (accel == XT_ACCEL_OCTREE) {
         // 16 resident 64-lane blocks per CU (LDS: 20 KB each)
         const unsigned g = (unsigned)std::min<size_t>(B.cap / XT_OCT_BLOCK + 1, (size_t)d->n_cu * 16);
-        hipLaunchKernelGGL((k_trace<XT_ACCEL_OCTREE, 1, XT_OCT_BLOCK>), dim3(g), dim3(XT_OCT_BLOCK), 0, st,
+        hipLaunchKernelGGL(k_trace_oct, dim3(g), dim3(XT_OCT_BLOCK), 0, st,
                            ds.view, B.q, B.count, B.hit, B.retest, B.recheck, B.cnt,
                            tn.trace_segments == XT_TRACE_SEGMENTS ? XT_TRACE_SEGMENTS : 1u);
     } else {

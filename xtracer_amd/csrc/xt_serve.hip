@@ -622,6 +622,9 @@ int regen_init(xt_dev *d, ServeState &S) {
     std::memset(R.ls_host, 0, sizeof R.ls_host);
     hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(align256(sz[4]) / 4, 256, 64)), dim3(256), 0, d->stream,
                        (uint32_t *)V.ctl, 0u, align256(sz[4]) / 4);
+    // the device-fed intake reads every entry's state, those never admitted too
+    hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(align256(sz[2]) / 4, 256, 64)), dim3(256), 0, d->stream,
+                       (uint32_t *)V.jobs, 0u, align256(sz[2]) / 4);
     hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(2ull * XT_REGEN_MAX_JOBS, 256, 64)), dim3(256), 0, d->stream,
                        (uint32_t *)V.done, 0u, 2ull * XT_REGEN_MAX_JOBS);
     hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(2ull * XT_REGEN_MAX_JOBS * XT_REGEN_SHARDS, 256, 512)), dim3(256), 0,

@@ -70,6 +70,7 @@ struct xt_dev {
     WaveBuffers wave;
     AccumBuffers accum;
     Counters *host_counters = nullptr;  // pinned, XT_MAX_LANES blocks
+    uint64_t *host_words = nullptr;     // pinned, 8 KiB: read-backs of an index build
     uint32_t *host_snap = nullptr;      // pinned, 2 x XT_MAX_LANES queue counts of the early-stop check
     hipEvent_t snap_ev[2][XT_MAX_LANES] = {};
     hipEvent_t ev0 = nullptr, ev1 = nullptr;

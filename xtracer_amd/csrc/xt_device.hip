@@ -61,6 +61,35 @@ int upload(xt_dev *d, T **p, const std::vector<T> &v, std::vector<void *> *track
     return XT_OK;
 }
 
+// Arrays uploaded into one device block (an allocation takes up to 0.7 ms, its
+// release as much): put() names them, place() allocates and copies.
+class Uploads {
+  public:
+    template <class T>
+    void put(T **p, const std::vector<T> &v) {
+        items.push_back({(void **)p, v.data(), v.size() * sizeof(T), total});
+        total += (std::max<size_t>(1, v.size()) * sizeof(T) + 255) & ~(size_t)255;
+    }
+    int place(xt_dev *d, std::vector<void *> *track, uint64_t *bytes) {
+        char *b = nullptr;
+        int rc = dev_alloc(d, &b, total, track, bytes);
+        if (rc) return rc;
+        for (const Item &i : items) {
+            *i.p = b + i.at;
+            if (i.bytes) XT_TRY(hipMemcpy(*i.p, i.src, i.bytes, hipMemcpyHostToDevice));
+        }
+        return XT_OK;
+    }
+
+  private:
+    struct Item {
+        void **p;
+        const void *src;
+        size_t bytes, at;
+    };
+    std::vector<Item> items;
+    size_t total = 0;
+};
 
 }  // namespace
 
@@ -180,6 +209,7 @@ void xt_dev_destroy(xt_dev *d) {
     xt_dev_free_accum(d);
     if (d->host_counters) hipHostFree(d->host_counters);
     if (d->host_snap) hipHostFree(d->host_snap);
+    if (d->host_words) hipHostFree(d->host_words);
     for (auto &row : d->snap_ev)
         for (hipEvent_t e : row)
             if (e) hipEventDestroy(e);
@@ -328,10 +358,28 @@ int xt_scene_upload(xt_dev *d, const xt_scene *s, uint32_t *scene_id) {
     if (mv.empty()) mv.push_back(XtMaterial{});
     std::vector<uint32_t> ms = f.mat_smp;
     ms.resize(3 * mv.size(), XT_NONE);  // the stand-in material samples nothing
-    int rc = upload(d, &prims, f.prims, t, b);
-    rc = rc ? rc : upload(d, &p64, f.prims64, t, b);
-    rc = rc ? rc : upload(d, &planes, f.planes, t, b);
+    if (f.tc64.size() != 6 * f.prims.size() || f.obj_uv_scale.size() != 2 * f.objects.size()) {
+        d->err = "texture coordinate arrays do not match the primitives";
+        return XT_E_SCENE;
+    }
+    Uploads up;
+    up.put(&prims, f.prims);
+    up.put(&p64, f.prims64);
+    up.put(&planes, f.planes);
+    up.put(&oct, f.oct_nodes);
+    up.put(&octr, f.oct_refs);
+    up.put(&om, obj_mat);
+    up.put(&mats, mv);
+    up.put(&tc64, f.tc64);
+    up.put(&obj_uv, f.obj_uv_scale);
+    up.put(&texels, f.texels);
+    up.put(&texs, f.textures);
+    up.put(&smps, f.samplers);
+    up.put(&msmp, ms);
+    if (!f.vnormals.empty()) up.put(&vn, f.vnormals);
+    int rc = up.place(d, t, b);
     if (!f.kd_deferred) {
+        // blocks of their own: a later build on the device replaces them
         const std::vector<XtKdNode> kdn = d->tuning.kd_layout == 2 ? xt::kd_line_layout(f.kd.nodes) : f.kd.nodes;
         rc = rc ? rc : upload(d, &kd, kdn, t, b);
         rc = rc ? rc : upload(d, &kdr, f.kd.refs, t, b);
@@ -341,21 +389,6 @@ int xt_scene_upload(xt_dev *d, const xt_scene *s, uint32_t *scene_id) {
         ds.n_kd_nodes = (uint32_t)std::max<size_t>(1, kdn.size());
         ds.n_kd_refs = (uint32_t)f.kd.refs.size();
     }
-    rc = rc ? rc : upload(d, &oct, f.oct_nodes, t, b);
-    rc = rc ? rc : upload(d, &octr, f.oct_refs, t, b);
-    rc = rc ? rc : upload(d, &om, obj_mat, t, b);
-    rc = rc ? rc : upload(d, &mats, mv, t, b);
-    if (!rc && (f.tc64.size() != 6 * f.prims.size() || f.obj_uv_scale.size() != 2 * f.objects.size())) {
-        d->err = "texture coordinate arrays do not match the primitives";
-        rc = XT_E_SCENE;
-    }
-    rc = rc ? rc : upload(d, &tc64, f.tc64, t, b);
-    rc = rc ? rc : upload(d, &obj_uv, f.obj_uv_scale, t, b);
-    rc = rc ? rc : upload(d, &texels, f.texels, t, b);
-    rc = rc ? rc : upload(d, &texs, f.textures, t, b);
-    rc = rc ? rc : upload(d, &smps, f.samplers, t, b);
-    rc = rc ? rc : upload(d, &msmp, ms, t, b);
-    if (!rc && !f.vnormals.empty()) rc = upload(d, &vn, f.vnormals, t, b);
     if (rc) {
         for (void *p : ds.allocs) hipFree(p);
         d->used -= std::min<uint64_t>(d->used, ds.bytes);

@@ -14,6 +14,7 @@
 #include "capi_internal.h"
 #include "device/xt_kdbuild.h"
 #include "xt_device.h"
+#include "xt_scratch.h"
 
 #define XT_TRY(expr)                                                                  \
     do {                                                                              \
@@ -41,41 +42,22 @@ struct Buf {
     size_t bytes = 0;
 };
 
-// Device memory of one build; everything still held is freed (after the
-// stream has drained) when the build ends.
+// The arrays of one build, in scratch memory.
 struct Work {
     xt_dev *d;
-    std::vector<Buf *> held;
-    explicit Work(xt_dev *dev) : d(dev) {}
-    ~Work() {
-        (void)hipStreamSynchronize(d->stream);
-        for (Buf *b : held)
-            if (b->p) {
-                (void)hipFree(b->p);
-                d->used -= std::min<uint64_t>(d->used, b->bytes);
-                b->p = nullptr;
-                b->bytes = 0;
-            }
-    }
+    XtScratch mem;
+    Work(xt_dev *dev, size_t block_bytes, bool exact) : d(dev), mem(dev, block_bytes, exact) {}
     // At least `need` bytes in b; `keep` copies the old contents over.
     int reserve(Buf &b, size_t need, bool keep) {
-        if (std::find(held.begin(), held.end(), &b) == held.end()) held.push_back(&b);
         if (need == 0) need = 256;
         if (need <= b.bytes) return XT_OK;
-        size_t nb = std::max(need, b.bytes + b.bytes / 2);
-        nb = (nb + 255) & ~(size_t)255;
-        if (d->budget && d->used + nb > d->budget) {
-            d->err = "device kd-tree build exceeds the HBM budget";
-            return XT_E_BUDGET;
-        }
+        const size_t nb = XtScratch::round(std::max(need, b.bytes + b.bytes / 2));
         void *p = nullptr;
-        XT_TRY(hipMalloc(&p, nb));
-        d->used += nb;
+        int rc = mem.take(&p, nb);
+        if (rc) return rc;
         if (b.p) {
             if (keep) XT_TRY(hipMemcpyAsync(p, b.p, b.bytes, hipMemcpyDeviceToDevice, d->stream));
-            XT_TRY(hipStreamSynchronize(d->stream));
-            (void)hipFree(b.p);
-            d->used -= std::min<uint64_t>(d->used, b.bytes);
+            mem.give(b.p, b.bytes);
         }
         b.p = p;
         b.bytes = nb;
@@ -114,7 +96,7 @@ struct KdOut {
     XtKdNode *nodes = nullptr;
     uint32_t *refs = nullptr;
     float4 *leaf = nullptr;
-    uint64_t nodes_bytes = 0, refs_bytes = 0, leaf_bytes = 0;
+    uint64_t nodes_bytes = 0, leaf_bytes = 0;  // nodes: the references' too, which follow in the same block
     float bounds[6] = {0, 0, 0, 0, 0, 0};
     xt_kd_build_stats stats{};
 };
@@ -131,8 +113,7 @@ int out_alloc(xt_dev *d, void **p, uint64_t bytes) {
 }
 
 void out_free(xt_dev *d, KdOut &o) {
-    for (auto pr : {std::make_pair((void *)o.nodes, o.nodes_bytes), std::make_pair((void *)o.refs, o.refs_bytes),
-                    std::make_pair((void *)o.leaf, o.leaf_bytes)})
+    for (auto pr : {std::make_pair((void *)o.nodes, o.nodes_bytes), std::make_pair((void *)o.leaf, o.leaf_bytes)})
         if (pr.first) {
             (void)hipFree(pr.first);
             d->used -= std::min<uint64_t>(d->used, pr.second);
@@ -140,7 +121,7 @@ void out_free(xt_dev *d, KdOut &o) {
     o = KdOut();
 }
 
-int build(xt_dev *d, const SceneView &v, const xt_build_params *bp, KdOut &o) {
+int build(xt_dev *d, const SceneView &v, const xt_build_params *bp, bool exact, KdOut &o) {
     const uint32_t n = v.n_prims;
     KdbParams P;
     xt::KdParams host;  // the host build's defaults
@@ -165,22 +146,15 @@ int build(xt_dev *d, const SceneView &v, const xt_build_params *bp, KdOut &o) {
         }
     } evs{e0, e1};
     XT_TRY(hipEventRecord(e0, d->stream));
-    Readback *hr = nullptr;
-    XT_TRY(hipHostMalloc((void **)&hr, sizeof(Readback), hipHostMallocDefault));
-    struct Pinned {
-        Readback *p;
-        ~Pinned() { (void)hipHostFree(p); }
-    } pinned{hr};
+    if (!d->host_words) XT_TRY(hipHostMalloc((void **)&d->host_words, 8192, hipHostMallocDefault));
+    Readback *const hr = (Readback *)d->host_words;
 
     if (n == 0) {
         // the host build's empty tree: a root leaf without references
-        int rc = out_alloc(d, (void **)&o.nodes, 256);
+        int rc = out_alloc(d, (void **)&o.nodes, 512);
         if (!rc) {
-            o.nodes_bytes = 256;
-            rc = out_alloc(d, (void **)&o.refs, 256);
-        }
-        if (!rc) {
-            o.refs_bytes = 256;
+            o.nodes_bytes = 512;
+            o.refs = (uint32_t *)((char *)o.nodes + 256);
             rc = out_alloc(d, (void **)&o.leaf, 256);
         }
         if (!rc) o.leaf_bytes = 256;
@@ -201,7 +175,8 @@ int build(xt_dev *d, const SceneView &v, const xt_build_params *bp, KdOut &o) {
         return XT_OK;
     }
 
-    Work W(d);
+    // what the terrain's build holds at its largest level is 420 bytes a primitive
+    Work W(d, 512ull * n + (1u << 20), exact);
     Buf r0[2], r1[2], nodes[2], split, big_of, nflags, nscan, flags, scan, l0, l1, q0, q1, tiles, gbins, chunks, ctl,
         part, bounds, gnodes, pool;
     int rc = XT_OK;
@@ -352,11 +327,11 @@ int build(xt_dev *d, const SceneView &v, const xt_build_params *bp, KdOut &o) {
     XT_TRY(hipMemcpyAsync(pos.p, &root_init[0], 4, hipMemcpyHostToDevice, d->stream));
     XT_TRY(hipMemcpyAsync(pairpos.p, &root_init[1], 4, hipMemcpyHostToDevice, d->stream));
     XT_TRY(hipMemcpyAsync(refpos.p, &root_init[2], 4, hipMemcpyHostToDevice, d->stream));
-    o.nodes_bytes = (sizeof(XtKdNode) * ((uint64_t)total + 1) + 255) & ~255ull;
-    o.refs_bytes = (4ull * pool_total + 255) & ~255ull;
+    const uint64_t refs_at = (sizeof(XtKdNode) * ((uint64_t)total + 1) + 255) & ~255ull;
+    o.nodes_bytes = refs_at + ((4ull * pool_total + 255) & ~255ull);
     o.leaf_bytes = (48ull * pool_total + 255) & ~255ull;
     rc = out_alloc(d, (void **)&o.nodes, o.nodes_bytes);
-    if (!rc) rc = out_alloc(d, (void **)&o.refs, o.refs_bytes);
+    o.refs = (uint32_t *)((char *)o.nodes + refs_at);
     if (!rc) rc = out_alloc(d, (void **)&o.leaf, o.leaf_bytes);
     if (rc) {
         (void)hipStreamSynchronize(d->stream);
@@ -416,14 +391,14 @@ void drop_kd(xt_dev *d, DevScene &ds) {
 
 int xt_kd_build_into(xt_dev *d, DevScene &ds, const xt_build_params *p) {
     KdOut o;
-    int rc = build(d, ds.view, p, o);
+    int rc = build(d, ds.view, p, false, o);
+    if (rc == XT_E_BUDGET) rc = build(d, ds.view, p, true, o);
     if (rc) return rc;
     XT_TRY(hipStreamSynchronize(d->stream));
     drop_kd(d, ds);
     ds.allocs.push_back(o.nodes);
-    ds.allocs.push_back(o.refs);
     ds.allocs.push_back(o.leaf);
-    ds.kd_bytes = o.nodes_bytes + o.refs_bytes + o.leaf_bytes;
+    ds.kd_bytes = o.nodes_bytes + o.leaf_bytes;
     ds.bytes += ds.kd_bytes;
     ds.view.kd = o.nodes;
     ds.view.kd_refs = o.refs;

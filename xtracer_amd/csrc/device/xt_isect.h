@@ -19,6 +19,11 @@
 #define XT_GRAZE 1e-5f       // |cos| below which the FP32 test defers
 #define XT_TSMALL 1e-5f      // relative t below which the FP32 test defers
 #define XT_TIE 2e-6f         // relative t difference treated as a possible tie
+// The wide BVH's boxes are widened by this times the largest coordinate of
+// the ray's origin and the scene: the FP32 test of a triangle misplaces its
+// edges by up to 2.5e-7 of that, and a box that the ray passes by as much must
+// not keep the triangle from being tested.
+#define XT_W_SLACK 1e-6f
 #define XT_EPS64 1e-8        // nmath EPSILON (lib/nmath/precision.h:87-89)
 
 struct f3 {

@@ -741,13 +741,10 @@ static __global__ void k_kdb_place(const XtKdNode *gnodes, uint32_t base, uint32
 // Each leaf reference's primitive record with the soup index as object word
 // (the FP32 walk's leaf copies).
 static __global__ void k_kdb_leaf_copies(const float4 *prims, uint32_t n_prims, const uint32_t *refs, uint32_t n,
-                                         float4 *leaf, KdbCtl *ctl) {
+                                         float4 *leaf) {
     for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < n; r += gridDim.x * blockDim.x) {
         const size_t s = refs[r];
-        if (s >= n_prims) {
-            atomicOr(&ctl->error, 16u);
-            continue;
-        }
+        if (s >= n_prims) continue;
         leaf[3 * (size_t)r] = prims[3 * s];
         const float4 b = prims[3 * s + 1];
         leaf[3 * (size_t)r + 1] = make_float4(b.x, b.y, b.z, __uint_as_float((uint32_t)s));

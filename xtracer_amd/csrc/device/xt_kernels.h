@@ -516,6 +516,7 @@ static __global__ __launch_bounds__(XT_OCT_BLOCK) void k_trace_oct(const SceneVi
     }
 }
 
+#include "xt_trace_bvh.h"
 #include "xt_trace_kd.h"
 
 __device__ __forceinline__ uint32_t object_of(const SceneView &S, uint32_t p) {

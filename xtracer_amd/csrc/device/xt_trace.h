@@ -17,6 +17,9 @@ struct SceneView {
     const XtKdNode *kd;
     const uint32_t *kd_refs;
     const float4 *kd_leaf;  // 3 float4 per leaf reference: the XtPrim with the soup index as object word
+    const uint4 *bvh;        // wide BVH, 8 uint4 per node (XtWideNode), or null: the FP32 walk uses the kd-tree
+    const float4 *bvh_leaf;  // 3 float4 per BVH primitive, records like kd_leaf's, in the tree's order
+    const uint32_t *bvh_refs;  // soup index per BVH primitive
     const XtOctNode *oct;
     const uint32_t *oct_refs;
     const uint32_t *obj_material;

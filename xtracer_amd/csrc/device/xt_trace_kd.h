@@ -52,7 +52,7 @@ static __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(XT_KD
         if (nw == 0 || (more && 64 - nw >= XT_REFILL_IDLE)) {
             if (__builtin_amdgcn_ballot_w64(done)) {
                 bool mark = false, full = false;
-                if (done) finish_ray(S, in, hit, cnt, ri, o, origin, ok, best, mark, full);
+                if (done) finish_ray(S, in, hit, cnt, ri, o, origin, ok, best, S.prims, best.prim, mark, full);
                 const bool rf = mark && full, rc = mark && !full;
                 if (__builtin_amdgcn_ballot_w64(mark)) {
                     const uint32_t slot = wave_append(rf, &cnt->n[CNT_RETEST]);

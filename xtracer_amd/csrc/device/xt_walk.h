@@ -5,7 +5,7 @@
 
 #define XT_STRETCH_LOG 12   // log2 of the rays of a stretch
 #define XT_RUN_MAX 512u     // rays of the longest run a wave takes at once
-#define XT_REFILL_IDLE 32   // a wave takes new rays once this many lanes are idle
+#define XT_REFILL_IDLE 24   // a wave takes new rays once this many lanes are idle
 
 // Where a wave's rays come from. Wave w first takes rays [64 w, 64 w + 64);
 // the rays beyond 64 times the grid's waves are cut into stretches of 2^sh
@@ -102,9 +102,10 @@ __device__ __forceinline__ uint32_t rank_in(unsigned long long m) {
 // Writes a walked ray's hit: the closest triangle's t and barycentrics in
 // FP64, or the FP32 record of a ray whose deferred candidates the FP64
 // kernels decide; `mark` and `full` as k_recheck and k_retest take them.
+// recs[3 rec ..] is the closest primitive's record, if it is a primitive.
 __device__ __forceinline__ void finish_ray(const SceneView &S, const Queue &in, float4 *hit, Counters *cnt,
-                                           uint32_t ri, f3 o, uint32_t origin, bool ok, const Best &best, bool &mark,
-                                           bool &full) {
+                                           uint32_t ri, f3 o, uint32_t origin, bool ok, const Best &best,
+                                           const float4 *recs, uint32_t rec, bool &mark, bool &full) {
     const float4 b4 = in.r1[ri];
     const f3 d = mk(b4.x, b4.y, b4.z);
     if (!ok) atomicAdd(&cnt->trace_fail, 1ull);
@@ -114,10 +115,10 @@ __device__ __forceinline__ void finish_ray(const SceneView &S, const Queue &in, 
     full = !ok || best.c1 == XT_CAND_OVERFLOW;
     float ht = best.t, hu = 0.f, hv = 0.f;
     if (!mark && best.prim < S.n_prims && !(b4.w > 0.f && best.prim == origin)) {
-        const float4 a = S.prims[3 * best.prim], b = S.prims[3 * best.prim + 1];
+        const float4 *q = recs + 3 * (size_t)rec;
+        const float4 a = q[0];
         // the closest triangle's t and barycentrics in FP64
-        if (XT_PRIM_TYPE(__float_as_uint(a.w)) == XT_PRIM_TRIANGLE)
-            tri_hit64(o, d, a, b, S.prims[3 * best.prim + 2], ht, hu, hv);
+        if (XT_PRIM_TYPE(__float_as_uint(a.w)) == XT_PRIM_TRIANGLE) tri_hit64(o, d, a, q[1], q[2], ht, hu, hv);
     }
     hit[ri] = make_float4(ht, __uint_as_float(best.prim), hu, hv);
 }

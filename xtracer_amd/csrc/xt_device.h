@@ -18,6 +18,7 @@ struct DevScene {
     uint64_t bytes = 0;
     uint64_t kd_bytes = 0;            // of the kd nodes, references and leaf copies (in `allocs`)
     uint32_t n_kd_nodes = 0, n_kd_refs = 0;
+    uint32_t n_bvh_nodes = 0, bvh_depth = 0;  // wide BVH (view.bvh), 0 without one
     xt_kd_build_stats kd_stats{};     // of the last device build (zero for a host-built tree)
     bool pt_supported = true;
     bool materials_supported = true;
@@ -117,9 +118,17 @@ struct TraceBufs {
 };
 int xt_launch_trace_bufs(xt_dev *d, const DevScene &ds, int accel, const TraceBufs &B, const double *ray64,
                          uint32_t *flags, bool time_it, hipStream_t st);
+class XtScratch;
+
 // Builds the kd-tree of a resident scene on the device (xt_kdbuild.hip) and
 // replaces the scene's kd arrays with it.
-int xt_kd_build_into(xt_dev *d, DevScene &ds, const xt_build_params *p);
+int xt_kd_build_into(xt_dev *d, DevScene &ds, const xt_build_params *p, XtScratch &mem);
+// Builds the scene's wide BVH, unless its FP32 walk stays on the kd-tree
+// (view.bvh is null then). xt_bvhbuild.hip
+int xt_bvh_build_into(xt_dev *d, DevScene &ds, XtScratch &mem);
+// Copies the kd leaves' primitives into leaf order for a scene that is walked
+// on its kd-tree (xt_kdbuild.hip).
+int xt_kd_leaf_copies(xt_dev *d, DevScene &ds);
 void xt_serve_shutdown(xt_dev *d);
 bool xt_serve_uses_scene(const xt_dev *d, uint32_t scene_id);
 void xt_serve_forget_scene(xt_dev *d, uint32_t scene_id);

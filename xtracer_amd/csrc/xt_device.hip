@@ -12,6 +12,7 @@
 #include "capi_internal.h"
 #include "device/xt_kernels.h"
 #include "xt_device.h"
+#include "xt_scratch.h"
 
 #define XT_TRY(expr)                                                                  \
     do {                                                                              \
@@ -332,16 +333,7 @@ int xt_scene_upload(xt_dev *d, const xt_scene *s, uint32_t *scene_id) {
         uint32_t m = f.objects[i].material;
         if (m != XT_NO_MATERIAL && !f.material_supported[m]) ds.pt_supported = ds.materials_supported = false;
     }
-    // kd leaves' primitives copied in leaf order, the object word replaced
-    // by the soup index, so the FP32 traversal reads a leaf's records
-    // without going through the reference list (a tree left to the device
-    // build is made after the other arrays are resident)
-    std::vector<XtPrim> leaf(f.kd_deferred ? 0 : f.kd.refs.size());
-    for (size_t r = 0; r < f.kd.refs.size(); ++r) {
-        leaf[r] = f.prims[f.kd.refs[r]];
-        leaf[r].object = f.kd.refs[r];
-    }
-    XtPrim *prims = nullptr, *kdl = nullptr;
+    XtPrim *prims = nullptr;
     XtPrim64 *p64 = nullptr;
     XtPlane *planes = nullptr;
     XtKdNode *kd = nullptr;
@@ -383,9 +375,7 @@ int xt_scene_upload(xt_dev *d, const xt_scene *s, uint32_t *scene_id) {
         const std::vector<XtKdNode> kdn = d->tuning.kd_layout == 2 ? xt::kd_line_layout(f.kd.nodes) : f.kd.nodes;
         rc = rc ? rc : upload(d, &kd, kdn, t, b);
         rc = rc ? rc : upload(d, &kdr, f.kd.refs, t, b);
-        rc = rc ? rc : upload(d, &kdl, leaf, t, b);
-        const size_t nr = std::max<size_t>(1, f.kd.refs.size());
-        ds.kd_bytes = sizeof(XtKdNode) * std::max<size_t>(1, kdn.size()) + 4 * nr + sizeof(XtPrim) * nr;
+        ds.kd_bytes = sizeof(XtKdNode) * std::max<size_t>(1, kdn.size()) + 4 * std::max<size_t>(1, f.kd.refs.size());
         ds.n_kd_nodes = (uint32_t)std::max<size_t>(1, kdn.size());
         ds.n_kd_refs = (uint32_t)f.kd.refs.size();
     }
@@ -401,7 +391,6 @@ int xt_scene_upload(xt_dev *d, const xt_scene *s, uint32_t *scene_id) {
     v.planes = planes;
     v.kd = kd;
     v.kd_refs = kdr;
-    v.kd_leaf = (const float4 *)kdl;
     v.oct = oct;
     v.oct_refs = octr;
     v.obj_material = om;
@@ -429,15 +418,21 @@ int xt_scene_upload(xt_dev *d, const xt_scene *s, uint32_t *scene_id) {
         leaf.count = 0;
         XT_TRY(hipMemcpy(kd, &leaf, sizeof leaf, hipMemcpyHostToDevice));
     }
+    XtScratch mem(d, xt_build_block(v.n_prims), false);
     if (f.kd_deferred) {
         xt_build_params bp{f.kd_params.max_depth, f.kd_params.leaf_prims, f.kd_params.cost_intersect, 0, 0};
-        rc = xt_kd_build_into(d, ds, &bp);
-        if (rc) {
-            (void)hipStreamSynchronize(d->stream);
-            for (void *p : ds.allocs) hipFree(p);
-            d->used -= std::min<uint64_t>(d->used, ds.bytes);
-            return rc;
-        }
+        rc = xt_kd_build_into(d, ds, &bp, mem);
+    }
+    // the FP32 walk's index: the wide BVH, or the kd-tree with its leaves'
+    // primitives copied in leaf order (the object word replaced by the soup
+    // index, so that a leaf's records are read without the reference list)
+    if (!rc) rc = xt_bvh_build_into(d, ds, mem);
+    if (!rc && !v.bvh) rc = xt_kd_leaf_copies(d, ds);
+    if (rc) {
+        (void)hipStreamSynchronize(d->stream);
+        for (void *p : ds.allocs) hipFree(p);
+        d->used -= std::min<uint64_t>(d->used, ds.bytes);
+        return rc;
     }
     const uint32_t id = d->next_scene++;
     d->scenes[id] = std::move(ds);
@@ -488,6 +483,33 @@ static void launch_kd_trace_sb(unsigned per_cu, int n_cu, size_t cap, hipStream_
                        cnt, nseg);
 }
 
+template <int STACK, int BS>
+static void launch_bvh_trace_sb(unsigned per_cu, int n_cu, size_t cap, hipStream_t st, const SceneView &v,
+                                const Queue &q, const uint32_t *count, float4 *hit, uint32_t *retest, uint4 *recheck,
+                                Counters *cnt, uint32_t nseg) {
+    static int resident = 0;
+    if (per_cu == 0) {
+        if (resident == 0) {
+            int nb = 0;
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_trace_bvh<STACK, BS>, BS, 0) != hipSuccess || nb < 1)
+                nb = 1;
+            resident = nb;
+        }
+        per_cu = (unsigned)resident;
+    }
+    const size_t need = (cap + BS - 1) / BS;
+    const unsigned g = (unsigned)std::max<size_t>(1, std::min<size_t>(need, (size_t)n_cu * per_cu));
+    hipLaunchKernelGGL((k_trace_bvh<STACK, BS>), dim3(g), dim3(BS), 0, st, v, q, count, hit, retest, recheck, cnt, nseg);
+}
+
+template <int STACK>
+static void launch_bvh_trace_s(unsigned bs, unsigned per_cu, int n_cu, size_t cap, hipStream_t st, const SceneView &v,
+                               const Queue &q, const uint32_t *count, float4 *hit, uint32_t *retest, uint4 *recheck,
+                               Counters *cnt, uint32_t nseg) {
+    if (bs == 128) launch_bvh_trace_sb<STACK, 128>(per_cu, n_cu, cap, st, v, q, count, hit, retest, recheck, cnt, nseg);
+    else launch_bvh_trace_sb<STACK, 256>(per_cu, n_cu, cap, st, v, q, count, hit, retest, recheck, cnt, nseg);
+}
+
 template <int STACK>
 static void launch_kd_trace_s(unsigned bs, unsigned per_cu, int n_cu, size_t cap, hipStream_t st, const SceneView &v,
                               const Queue &q, const uint32_t *count, float4 *hit, uint32_t *retest, uint4 *recheck, Counters *cnt, uint32_t nseg) {
@@ -495,12 +517,20 @@ static void launch_kd_trace_s(unsigned bs, unsigned per_cu, int n_cu, size_t cap
     else launch_kd_trace_sb<STACK, 256>(per_cu, n_cu, cap, st, v, q, count, hit, retest, recheck, cnt, nseg);
 }
 
-static void launch_kd_trace(const xt_tuning &tn, int n_cu, size_t cap, hipStream_t st, const SceneView &view,
+static void launch_kd_trace(const xt_tuning &tn, uint32_t bvh_depth, int n_cu, size_t cap, hipStream_t st, const SceneView &view,
                             const Queue &q, const uint32_t *count, float4 *hit, uint32_t *retest, uint4 *recheck, Counters *cnt) {
     const uint32_t nseg = tn.trace_segments == XT_TRACE_SEGMENTS ? XT_TRACE_SEGMENTS : 1u;
     SceneView v = view;
     v.kd_indexed = tn.kd_leaf == 2;
     const unsigned bs = tn.trace_block, pc = tn.trace_blocks_per_cu;
+    if (v.bvh) {
+        // a walk holds a group for each level but the root's and the leaves'
+        const uint32_t s = bvh_depth < 2 ? 0 : bvh_depth - 2;
+        if (s <= 8) launch_bvh_trace_s<8>(bs, pc, n_cu, cap, st, v, q, count, hit, retest, recheck, cnt, nseg);
+        else if (s <= 12) launch_bvh_trace_s<12>(bs, pc, n_cu, cap, st, v, q, count, hit, retest, recheck, cnt, nseg);
+        else launch_bvh_trace_sb<24, 128>(pc, n_cu, cap, st, v, q, count, hit, retest, recheck, cnt, nseg);
+        return;
+    }
     switch (tn.kd_stack) {
         case 8: launch_kd_trace_s<8>(bs, pc, n_cu, cap, st, v, q, count, hit, retest, recheck, cnt, nseg); break;
         case 12: launch_kd_trace_s<12>(bs, pc, n_cu, cap, st, v, q, count, hit, retest, recheck, cnt, nseg); break;
@@ -523,7 +553,7 @@ int xt_launch_trace_bufs(xt_dev *d, const DevScene &ds, int accel, const TraceBu
                            ds.view, B.q, B.count, B.hit, B.retest, B.recheck, B.cnt,
                            tn.trace_segments == XT_TRACE_SEGMENTS ? XT_TRACE_SEGMENTS : 1u);
     } else {
-        launch_kd_trace(tn, d->n_cu, B.cap, st, ds.view, B.q, B.count, B.hit, B.retest, B.recheck, B.cnt);
+        launch_kd_trace(tn, ds.bvh_depth, d->n_cu, B.cap, st, ds.view, B.q, B.count, B.hit, B.retest, B.recheck, B.cnt);
     }
     if (timed) {
         hipEventRecord(d->tev[d->trace_launches + 1], st);

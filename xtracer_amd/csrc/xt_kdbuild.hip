@@ -45,8 +45,7 @@ struct Buf {
 // The arrays of one build, in scratch memory.
 struct Work {
     xt_dev *d;
-    XtScratch mem;
-    Work(xt_dev *dev, size_t block_bytes, bool exact) : d(dev), mem(dev, block_bytes, exact) {}
+    XtScratch &mem;
     // At least `need` bytes in b; `keep` copies the old contents over.
     int reserve(Buf &b, size_t need, bool keep) {
         if (need == 0) need = 256;
@@ -95,8 +94,7 @@ const char *kdb_error(uint32_t e) {
 struct KdOut {
     XtKdNode *nodes = nullptr;
     uint32_t *refs = nullptr;
-    float4 *leaf = nullptr;
-    uint64_t nodes_bytes = 0, leaf_bytes = 0;  // nodes: the references' too, which follow in the same block
+    uint64_t nodes_bytes = 0;  // with the references, which follow in the same block
     float bounds[6] = {0, 0, 0, 0, 0, 0};
     xt_kd_build_stats stats{};
 };
@@ -113,15 +111,14 @@ int out_alloc(xt_dev *d, void **p, uint64_t bytes) {
 }
 
 void out_free(xt_dev *d, KdOut &o) {
-    for (auto pr : {std::make_pair((void *)o.nodes, o.nodes_bytes), std::make_pair((void *)o.leaf, o.leaf_bytes)})
-        if (pr.first) {
-            (void)hipFree(pr.first);
-            d->used -= std::min<uint64_t>(d->used, pr.second);
-        }
+    if (o.nodes) {
+        (void)hipFree(o.nodes);
+        d->used -= std::min<uint64_t>(d->used, o.nodes_bytes);
+    }
     o = KdOut();
 }
 
-int build(xt_dev *d, const SceneView &v, const xt_build_params *bp, bool exact, KdOut &o) {
+int build(xt_dev *d, const SceneView &v, const xt_build_params *bp, XtScratch &mem, KdOut &o) {
     const uint32_t n = v.n_prims;
     KdbParams P;
     xt::KdParams host;  // the host build's defaults
@@ -152,16 +149,9 @@ int build(xt_dev *d, const SceneView &v, const xt_build_params *bp, bool exact, 
     if (n == 0) {
         // the host build's empty tree: a root leaf without references
         int rc = out_alloc(d, (void **)&o.nodes, 512);
-        if (!rc) {
-            o.nodes_bytes = 512;
-            o.refs = (uint32_t *)((char *)o.nodes + 256);
-            rc = out_alloc(d, (void **)&o.leaf, 256);
-        }
-        if (!rc) o.leaf_bytes = 256;
-        if (rc) {
-            out_free(d, o);
-            return rc;
-        }
+        if (rc) return rc;
+        o.nodes_bytes = 512;
+        o.refs = (uint32_t *)((char *)o.nodes + 256);
         static const XtKdNode leaves[2] = {{3u, {0.f}}, {3u, {0.f}}};  // the root and the padding leaf
         XT_TRY(hipMemcpyAsync(o.nodes, leaves, sizeof leaves, hipMemcpyHostToDevice, d->stream));
         XT_TRY(hipEventRecord(e1, d->stream));
@@ -175,8 +165,7 @@ int build(xt_dev *d, const SceneView &v, const xt_build_params *bp, bool exact, 
         return XT_OK;
     }
 
-    // what the terrain's build holds at its largest level is 420 bytes a primitive
-    Work W(d, 512ull * n + (1u << 20), exact);
+    Work W{d, mem};
     Buf r0[2], r1[2], nodes[2], split, big_of, nflags, nscan, flags, scan, l0, l1, q0, q1, tiles, gbins, chunks, ctl,
         part, bounds, gnodes, pool;
     int rc = XT_OK;
@@ -329,10 +318,8 @@ int build(xt_dev *d, const SceneView &v, const xt_build_params *bp, bool exact, 
     XT_TRY(hipMemcpyAsync(refpos.p, &root_init[2], 4, hipMemcpyHostToDevice, d->stream));
     const uint64_t refs_at = (sizeof(XtKdNode) * ((uint64_t)total + 1) + 255) & ~255ull;
     o.nodes_bytes = refs_at + ((4ull * pool_total + 255) & ~255ull);
-    o.leaf_bytes = (48ull * pool_total + 255) & ~255ull;
     rc = out_alloc(d, (void **)&o.nodes, o.nodes_bytes);
     o.refs = (uint32_t *)((char *)o.nodes + refs_at);
-    if (!rc) rc = out_alloc(d, (void **)&o.leaf, o.leaf_bytes);
     if (rc) {
         (void)hipStreamSynchronize(d->stream);
         out_free(d, o);
@@ -346,9 +333,6 @@ int build(xt_dev *d, const SceneView &v, const xt_build_params *bp, bool exact, 
                            as<uint32_t>(pos), as<uint32_t>(pairpos), as<uint32_t>(refpos),
                            (const uint32_t *)as<uint32_t>(pool), pool_total, total, o.nodes, total + 1, o.refs,
                            pool_total, as<KdbCtl>(ctl));
-    if (pool_total)
-        hipLaunchKernelGGL(k_kdb_leaf_copies, dim3(grid_for(pool_total, 256, 16384)), dim3(256), 0, d->stream,
-                           v.prims, n, (const uint32_t *)o.refs, pool_total, o.leaf, as<KdbCtl>(ctl));
     XT_LAUNCHED();
     XT_TRY(hipEventRecord(e1, d->stream));
     XT_TRY(hipMemcpyAsync(&hr->ctl, ctl.p, sizeof(KdbCtl), hipMemcpyDeviceToHost, d->stream));
@@ -389,20 +373,23 @@ void drop_kd(xt_dev *d, DevScene &ds) {
 
 }  // namespace
 
-int xt_kd_build_into(xt_dev *d, DevScene &ds, const xt_build_params *p) {
+int xt_kd_build_into(xt_dev *d, DevScene &ds, const xt_build_params *p, XtScratch &mem) {
     KdOut o;
-    int rc = build(d, ds.view, p, false, o);
-    if (rc == XT_E_BUDGET) rc = build(d, ds.view, p, true, o);
+    int rc = build(d, ds.view, p, mem, o);
+    mem.reset();
+    if (rc == XT_E_BUDGET) {
+        mem.release();
+        XtScratch exact(d, 0, true);
+        rc = build(d, ds.view, p, exact, o);
+    }
     if (rc) return rc;
     XT_TRY(hipStreamSynchronize(d->stream));
     drop_kd(d, ds);
     ds.allocs.push_back(o.nodes);
-    ds.allocs.push_back(o.leaf);
-    ds.kd_bytes = o.nodes_bytes + o.leaf_bytes;
+    ds.kd_bytes = o.nodes_bytes;
     ds.bytes += ds.kd_bytes;
     ds.view.kd = o.nodes;
     ds.view.kd_refs = o.refs;
-    ds.view.kd_leaf = o.leaf;
     for (int a = 0; a < 3; ++a) {
         ds.view.kb_lo[a] = o.bounds[a];
         ds.view.kb_hi[a] = o.bounds[3 + a];
@@ -410,6 +397,24 @@ int xt_kd_build_into(xt_dev *d, DevScene &ds, const xt_build_params *p) {
     ds.n_kd_nodes = o.stats.n_nodes;
     ds.n_kd_refs = o.stats.n_refs;
     ds.kd_stats = o.stats;
+    return XT_OK;
+}
+
+int xt_kd_leaf_copies(xt_dev *d, DevScene &ds) {
+    const uint64_t bytes = std::max<uint64_t>(256, sizeof(XtPrim) * (uint64_t)ds.n_kd_refs);
+    void *p = nullptr;
+    int rc = out_alloc(d, &p, bytes);
+    if (rc) return rc;
+    ds.allocs.push_back(p);
+    ds.bytes += bytes;
+    ds.kd_bytes += bytes;
+    ds.view.kd_leaf = (const float4 *)p;
+    if (ds.n_kd_refs) {
+        hipLaunchKernelGGL(k_kdb_leaf_copies, dim3(grid_for(ds.n_kd_refs, 256, 16384)), dim3(256), 0, d->stream,
+                           ds.view.prims, ds.view.n_prims, ds.view.kd_refs, ds.n_kd_refs, (float4 *)p);
+        XT_LAUNCHED();
+        XT_TRY(hipStreamSynchronize(d->stream));
+    }
     return XT_OK;
 }
 
@@ -430,7 +435,9 @@ int xt_scene_build_kd_device(xt_dev *d, uint32_t scene_id, const xt_build_params
     XT_TRY(hipSetDevice(d->device));
     XT_TRY(hipStreamSynchronize(d->stream));
     xt_serve_forget_scene(d, scene_id);  // idle serving lanes hold the scene's old arrays
-    int rc = xt_kd_build_into(d, it->second, p);
+    XtScratch mem(d, xt_build_block(it->second.view.n_prims), false);
+    int rc = xt_kd_build_into(d, it->second, p, mem);
+    if (!rc && !it->second.view.bvh) rc = xt_kd_leaf_copies(d, it->second);
     if (rc) return rc;
     if (stats) *stats = it->second.kd_stats;
     return XT_OK;

@@ -107,6 +107,34 @@ struct XtKdNode {
     };
 };
 
+// Wide BVH node, 128 bytes (one L2 line): up to eight children, each an inner
+// node or a leaf of 1 to 4 primitives, with boxes on an integer grid of the
+// node's own (after Ylitie, Karras, Laine, "Efficient Incoherent Ray Traversal
+// on GPUs Through Compressed Wide BVHs", HPG 2017, with 16-bit floats for the
+// planes, which the FP32 fused multiply-add takes as they are). Child slot s
+// is meant for children lying towards the corner of the node whose axis signs
+// are the bits of s, so that visiting slots by s ^ (ray sign bits) goes
+// roughly front to back.
+struct XtWideNode {
+    float p[3];          // grid origin
+    float step;          // grid step of all axes
+    uint32_t child;      // node of slot 0; the inner child of slot s is node child + s
+    uint32_t prims;      // first primitive of the node's leaves (they follow each other in slot order)
+    uint32_t masks;      // slots: leaves (bits 0-7), bits 0 and 1 of their primitive count - 1 (8-15, 16-23), inner (24-31)
+    uint32_t pad;
+    uint16_t plane[6][8];  // lower x, y, z, upper x, y, z of each slot: binary16 integers 0..2047
+};
+#define XT_WIDE_MAX_NODES (1u << 24)
+#define XT_WIDE_LEAF 4u
+#define XT_WIDE_GRID 2047.f
+// Scenes whose primitives fill their boxes worse than this (sum of the boxes'
+// half areas over the primitives' areas) keep the kd-tree walk, whose leaves
+// clip them: a ray meets too many boxes of long thin slanting triangles. Meshes
+// lie at 3.4 (icosphere, terrain: frames in 0.53 to 0.69 of the kd-tree walk's
+// time), the hair strands at 33 (1024x1024, 8 samples: 24.5 ms with the kd-tree
+// walk, 56.2 ms with the BVH).
+#define XT_BVH_MAX_BOX_RATIO 12.0
+
 // Octree node in breadth-first order (children of a node are 8 consecutive
 // nodes). Box rounded outward to FP32. Items are a contiguous range of the
 // soup because the soup is laid out in the octree's pre-order.
@@ -126,5 +154,6 @@ static_assert(sizeof(XtPrim64) == 72, "XtPrim64 layout");
 static_assert(sizeof(XtPlane) == 80, "XtPlane layout");
 static_assert(sizeof(XtMaterial) == 48, "XtMaterial layout");
 static_assert(sizeof(XtKdNode) == 8, "XtKdNode layout");
+static_assert(sizeof(XtWideNode) == 128, "XtWideNode layout");
 static_assert(sizeof(XtOctNode) == 48, "XtOctNode layout");
 #endif

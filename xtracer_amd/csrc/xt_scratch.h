@@ -25,10 +25,18 @@ class XtScratch {
     XtScratch(xt_dev *dev, size_t block_bytes, bool exact_) : exact(exact_), d(dev), block(block_bytes) {}
     XtScratch(const XtScratch &) = delete;
     XtScratch &operator=(const XtScratch &) = delete;
-    ~XtScratch() {
+    ~XtScratch() { release(); }
+    // Every range back; the blocks are kept.
+    void reset() {
+        if (exact) return release();
+        for (Block &b : blocks) b.free = {{0, b.bytes}};
+    }
+    // Every range back and the blocks freed.
+    void release() {
         if (blocks.empty()) return;
         (void)hipStreamSynchronize(d->stream);
         for (Block &b : blocks) drop(b);
+        blocks.clear();
     }
     const bool exact;
 
@@ -48,6 +56,7 @@ class XtScratch {
         Block b;
         b.bytes = exact ? bytes : std::max(bytes, round(block));
         block = std::max<size_t>(block / 2, 1u << 20);
+        if (d->budget && d->used + b.bytes > d->budget) b.bytes = bytes;
         if (d->budget && d->used + b.bytes > d->budget) {
             d->err = "device build exceeds the HBM budget";
             return XT_E_BUDGET;
@@ -109,3 +118,7 @@ class XtScratch {
     size_t block;  // bytes of the next block
     std::vector<Block> blocks;
 };
+
+// The first block of a scene's index builds: the kd-tree build of the terrain
+// holds 420 bytes a primitive at its largest level, a wide BVH build 400.
+inline size_t xt_build_block(uint32_t n_prims) { return 512ull * n_prims + (1u << 21); }

@@ -19,25 +19,37 @@
 
 #define XT_BLOCK 256
 #define XT_OCT_BLOCK 64
+#define XT_RECHECK_BLOCK 64
 #define XT_TRACE_CHUNK 1  // 64-ray groups a trace wave takes per cursor fetch
 #define XT_DEAD 0xfffffffeu  // origin word of a queue entry without a ray
 
 // Indices into the device counter block.
 enum {
-    CNT_Q0 = 0,      // ray count of queue 0
-    CNT_Q1 = 1,      // ray count of queue 1
-    CNT_RETEST = 2,  // rays listed for the FP64 re-test
-    CNT_CURSOR = 3,  // work cursor of the persistent trace kernel
-    CNT_RECHECK = 4, // rays listed for the FP64 re-check of their deferred candidates
+    CNT_Q0 = 0,       // ray count of queue 0
+    CNT_Q1 = 1,       // ray count of queue 1
+    CNT_RETEST = 2,   // + parity: rays listed for the FP64 re-test
+    CNT_RECHECK = 4,  // + parity: rays listed for the FP64 re-check of their deferred candidates
     CNT_WORDS = 8
 };
 #define XT_TRACE_SEGMENTS 8  // XCDs of an MI355X: one trace-queue segment each
 #define XT_CURSOR_STRIDE 32
+// A query round has a parity, the index of the queue it reads: it counts in
+// its parity's lists and cursors, and its trace clears the other parity's, and
+// the other queue's count, for the round after it, so that rounds need no
+// clearing launch of their own.
 struct Counters {
     uint32_t n[CNT_WORDS];
-    uint32_t seg[XT_TRACE_SEGMENTS];  // work cursors of the trace queue's segments (reset with CNT_CURSOR)
     unsigned long long queries, retests, steps_exceeded, trace_fail;
-    uint32_t xcd[XT_TRACE_SEGMENTS * XT_CURSOR_STRIDE];  // work cursors, one L2 line each (reset with CNT_CURSOR)
+    uint32_t cursor[2][XT_TRACE_SEGMENTS * XT_CURSOR_STRIDE];  // work cursors, one L2 line each
+};
+
+// What a trace launch counts in and reports to.
+struct TraceCtl {
+    Counters *cnt;
+    uint32_t par;     // parity of the round
+    uint32_t nseg;    // segments of the queue
+    uint64_t *stamp;  // or null: wall clock of the trace's start; stamp[1]: of its end (pinned host memory)
+    uint32_t *post;   // or null: the queue's ray count (pinned host memory)
 };
 
 struct Queue {
@@ -104,33 +116,29 @@ __device__ __forceinline__ bool slot_pixel(const JobDev &j, uint32_t q, uint32_t
     return x < j.W && y < j.H;
 }
 
-static __global__ void k_reset(Counters *c, uint32_t mask) {
+// Everything of a counter block to zero, but the count of queue 0.
+__device__ __forceinline__ void reset_counters(Counters *c, uint32_t rays, bool totals) {
     const uint32_t i = threadIdx.x;
-    if (i < CNT_WORDS && (mask >> i) & 1u) c->n[i] = 0;
-    if (i < XT_TRACE_SEGMENTS && (mask >> CNT_CURSOR) & 1u) c->seg[i] = c->xcd[i * XT_CURSOR_STRIDE] = 0;
-    if (i == 0 && (mask >> 31) & 1u) {
-        c->queries = 0;
-        c->retests = 0;
-        c->steps_exceeded = 0;
-        c->trace_fail = 0;
-    }
+    if (i < CNT_WORDS) c->n[i] = i == CNT_Q0 ? rays : 0u;
+    if (i < 2 * XT_TRACE_SEGMENTS) c->cursor[i >> 3][(i & 7u) * XT_CURSOR_STRIDE] = 0;
+    if (i == 0 && totals) c->queries = c->retests = c->steps_exceeded = c->trace_fail = 0;
 }
 
-// k_reset over `gridDim.x` consecutive counter blocks (one per lane).
-static __global__ void k_reset_lanes(Counters *c, uint32_t mask) {
-    Counters *b = c + blockIdx.x;
-    const uint32_t i = threadIdx.x;
-    if (i < CNT_WORDS && (mask >> i) & 1u) b->n[i] = 0;
-    if (i < XT_TRACE_SEGMENTS && (mask >> CNT_CURSOR) & 1u) b->seg[i] = b->xcd[i * XT_CURSOR_STRIDE] = 0;
-    if (i == 0 && (mask >> 31) & 1u) {
-        b->queries = 0;
-        b->retests = 0;
-        b->steps_exceeded = 0;
-        b->trace_fail = 0;
-    }
-}
+// One counter block per workgroup.
+static __global__ void k_reset(Counters *c, uint32_t rays) { reset_counters(c + blockIdx.x, rays, true); }
 
-static __global__ void k_set_count(Counters *c, uint32_t which, uint32_t value) { c->n[which] = value; }
+// The start of a trace over n rays: every block calls it, block 0 acts.
+__device__ __forceinline__ void trace_open(const TraceCtl &T, uint32_t n) {
+    if (blockIdx.x != 0) return;
+    const uint32_t t = threadIdx.x, other = T.par ^ 1u;
+    if (t == 0) {
+        if (T.stamp) *T.stamp = wall_clock64();
+        if (T.post) __hip_atomic_store(T.post, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        T.cnt->queries += n;
+        T.cnt->n[CNT_Q0 + other] = T.cnt->n[CNT_RETEST + other] = T.cnt->n[CNT_RECHECK + other] = 0;
+    }
+    if (t < XT_TRACE_SEGMENTS) T.cnt->cursor[other][t * XT_CURSOR_STRIDE] = 0;
+}
 
 static __global__ void k_fill_u32(uint32_t *p, uint32_t value, size_t n) {
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
@@ -342,12 +350,14 @@ __device__ __forceinline__ void aa_coords(const JobDev &j, uint32_t px, uint32_t
 // the image edge, samples past the job's count) get a dead ray, which the
 // trace turns into a miss whose radiance is never accumulated. The path
 // state word ps1.w holds the query count (low 16 bits) and the job's rdepth
-// (high 16 bits).
+// (high 16 bits). cnt, when given, is the lane's counter block, set up for the
+// pass (its totals with the first).
 static __global__ __launch_bounds__(XT_BLOCK) void k_camera(const JobDev j, uint32_t pass_base, uint32_t spp_pass,
                                                      uint32_t q0, uint32_t qn, uint32_t path_base, Queue out,
                                                      float4 *ps0, float4 *ps1, float4 *rad, double *ray64,
-                                                     uint32_t order) {
+                                                     uint32_t order, Counters *cnt) {
     const uint32_t n = spp_pass * qn;
+    if (cnt && blockIdx.x == 0) reset_counters(cnt, n, pass_base == 0);
     const uint32_t stride = gridDim.x * blockDim.x;
     const uint32_t qword = 1u | (j.rdepth << 16);
     // order 2 (with whole tiles): queue entry i holds sample sl of slot w of
@@ -437,11 +447,13 @@ __device__ __forceinline__ uint32_t seg_begin(uint32_t n, uint32_t s, uint32_t n
 // others.
 static __global__ __launch_bounds__(XT_OCT_BLOCK) void k_trace_oct(const SceneView S, const Queue in,
                                                             const uint32_t *in_count, float4 *hit,
-                                                            uint32_t *retest_list, uint4 *recheck_list, Counters *cnt,
-                                                            uint32_t nseg) {
+                                                            uint32_t *retest_list, uint4 *recheck_list,
+                                                            const TraceCtl T) {
+    Counters *const cnt = T.cnt;
+    const uint32_t nseg = T.nseg;
     __shared__ uint32_t ostk[XT_OCT_STACK * XT_OCT_BLOCK];
     const uint32_t n = *in_count;
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&cnt->queries, (unsigned long long)n);
+    trace_open(T, n);
     const uint32_t lane = lane_id();
     uint32_t chunk = 0, part = XT_TRACE_CHUNK;
     uint32_t seg = blockIdx.x % nseg, tried = 0;
@@ -453,7 +465,7 @@ static __global__ __launch_bounds__(XT_OCT_BLOCK) void k_trace_oct(const SceneVi
                 // the loop ends
                 while (tried < nseg) {
                     const uint32_t lo = seg_begin(n, seg, nseg), hi = seg_begin(n, seg + 1, nseg);
-                    const uint32_t c = atomicAdd(&cnt->seg[seg], 64u * XT_TRACE_CHUNK);
+                    const uint32_t c = atomicAdd(&cnt->cursor[T.par][seg * XT_CURSOR_STRIDE], 64u * XT_TRACE_CHUNK);
                     if (c < hi - lo) {
                         chunk = lo + c;
                         break;
@@ -509,9 +521,9 @@ static __global__ __launch_bounds__(XT_OCT_BLOCK) void k_trace_oct(const SceneVi
         // rays with a few deferred candidates get the FP64 re-check of just
         // those; rays with more, or whose traversal gave up, the full re-test
         const bool rf = mark && full, rc = mark && !full;
-        const uint32_t slot = wave_append(rf, &cnt->n[CNT_RETEST]);
+        const uint32_t slot = wave_append(rf, &cnt->n[CNT_RETEST + T.par]);
         if (rf) retest_list[slot] = i;
-        const uint32_t cslot = wave_append(rc, &cnt->n[CNT_RECHECK]);
+        const uint32_t cslot = wave_append(rc, &cnt->n[CNT_RECHECK + T.par]);
         if (rc) recheck_list[cslot] = make_uint4(i, c0, c1, XT_NONE);
     }
 }
@@ -523,22 +535,38 @@ __device__ __forceinline__ uint32_t object_of(const SceneView &S, uint32_t p) {
     return p >= XT_PLANE_BASE ? S.planes[p - XT_PLANE_BASE].object : __float_as_uint(S.prims[3 * p + 1].w);
 }
 
-// FP64 re-check of a ray's FP32 closest hit and its deferred candidates: the
-// reference's predicates (triangle.cc:82-123, sphere.cc:35-61,
-// plane.cc:19-61) on those primitives alone, ordered by (t, object, soup
-// index) like Scene::intersection. The FP32 traversal stopped at its closest
-// hit, so when the FP64 winner lies beyond it (or the FP32 closest hit is
-// rejected and nothing else hits) the ray goes on to the full re-test.
-static __global__ __launch_bounds__(XT_BLOCK) void k_recheck(const SceneView S, const Queue in, float4 *hit,
-                                                        const uint4 *list, uint32_t *retest_list, Counters *cnt,
-                                                        const double *ray64, uint32_t *flags) {
-    const uint32_t n = cnt->n[CNT_RECHECK];
-    const uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += stride) {
+// The FP64 kernel behind a trace. First the listed rays with a few deferred
+// candidates: the FP32 closest hit and the candidates under the reference's
+// predicates (triangle.cc:82-123, sphere.cc:35-61, plane.cc:19-61) alone,
+// ordered by (t, object, soup index) like Scene::intersection. The FP32
+// traversal stopped at its closest hit, so when the FP64 winner lies beyond it
+// (or the FP32 closest hit is rejected and nothing else hits) the ray takes
+// the full re-test, as do the rays listed for it: the FP64 walk. ray64
+// (optional) holds the FP64 rays by path id; otherwise the FP32 ray is widened.
+// One launch for both lists: usually few rays or none (1 in 13,000 of the 1080p
+// icosphere frame is re-checked, 3 of 78 M re-tested), and a launch costs about
+// 4 us. Bound by the longest FP64 walk. One-wave blocks: the 50 KB of stacks of
+// a four-wave block wait for a compute unit that a trace of another group has
+// left (hair strands frame 24.4 ms, with one-wave blocks 23.6).
+template <int ACCEL>
+static __global__ __launch_bounds__(XT_RECHECK_BLOCK) void k_recheck(
+    const SceneView S, const Queue in, float4 *hit, const uint4 *list, const uint32_t *retest_list, const TraceCtl T,
+    const double *ray64, uint32_t *flags) {
+    constexpr int BS = XT_RECHECK_BLOCK;
+    __shared__ uint2 kstk[ACCEL == XT_ACCEL_KDTREE ? (XT_KD_STACK + 1) * BS : 1];
+    __shared__ uint32_t ostk[ACCEL == XT_ACCEL_OCTREE ? XT_OCT_STACK * BS : 1];
+    Counters *const cnt = T.cnt;
+    const uint32_t nc = cnt->n[CNT_RECHECK + T.par], nt = cnt->n[CNT_RETEST + T.par], n = nc + nt;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (T.stamp) T.stamp[1] = wall_clock64();
+        if (nt) atomicAdd(&cnt->retests, (unsigned long long)nt);
+    }
+    const uint32_t stride = gridDim.x * BS;
+    for (uint32_t base = blockIdx.x * BS; base < n; base += stride) {
         const uint32_t k = base + threadIdx.x;
         bool need = false;
         uint32_t i = 0;
-        if (k < n) {
+        if (k < nc) {
             const uint4 e = list[k];
             i = e.x;
             const float4 a = in.r0[i], b = in.r1[i];
@@ -576,34 +604,18 @@ static __global__ __launch_bounds__(XT_BLOCK) void k_recheck(const SceneView S, 
             // of space when it found none)
             if (B != XT_NONE && !(tst.bt <= (double)h.x * (1.0 + 4.0 * XT_TIE))) {
                 need = true;
+                atomicAdd(&cnt->retests, 1ull);
             } else {
                 const bool is_tri = tst.prim < S.n_prims;
                 hit[i] = make_float4(tst.prim == XT_NONE ? INFINITY : (float)tst.bt, __uint_as_float(tst.prim),
                                      is_tri ? (float)tst.b1 : 0.f, is_tri ? (float)tst.b2 : 0.f);
                 if (flags) flags[i] |= 1u;
             }
+        } else if (k < n) {
+            need = true;
+            i = retest_list[k - nc];
         }
-        const uint32_t slot = wave_append(need, &cnt->n[CNT_RETEST]);
-        if (need) retest_list[slot] = i;
-    }
-}
-
-// FP64 re-test of listed rays. ray64 (optional) holds the FP64 rays by path
-// id; otherwise the FP32 ray is widened.
-template <int ACCEL>
-static __global__ __launch_bounds__(ACCEL == XT_ACCEL_KDTREE ? XT_BLOCK : XT_OCT_BLOCK) void k_retest(
-    const SceneView S, const Queue in, float4 *hit, const uint32_t *list, Counters *cnt, const double *ray64,
-    uint32_t *flags) {
-    constexpr int BS = ACCEL == XT_ACCEL_KDTREE ? XT_BLOCK : XT_OCT_BLOCK;
-    __shared__ uint2 kstk[ACCEL == XT_ACCEL_KDTREE ? (XT_KD_STACK + 1) * XT_BLOCK : 1];
-    __shared__ uint32_t ostk[ACCEL == XT_ACCEL_OCTREE ? XT_OCT_STACK * XT_OCT_BLOCK : 1];
-    const uint32_t n = cnt->n[CNT_RETEST];
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&cnt->retests, (unsigned long long)n);
-    const uint32_t stride = gridDim.x * BS;
-    for (uint32_t base = blockIdx.x * BS; base < n; base += stride) {
-        const uint32_t k = base + threadIdx.x;
-        if (k >= n) continue;
-        const uint32_t i = list[k];
+        if (!need) continue;
         const float4 a = in.r0[i], b = in.r1[i];
         RayF r;
         r.o = mk(a.x, a.y, a.z);
@@ -1207,22 +1219,50 @@ __device__ __forceinline__ void neumaier_add(double2 &a, double x) {
 }
 #pragma clang fp contract(on)
 
+// A pixel's image value from its float sum or its compensated FP64 sums.
+__device__ __forceinline__ float4 resolve_px(const JobDev &j, float4 a, double2 s0, double2 s1, double2 s2) {
+    if (j.accum == XT_ACCUM_REFERENCE) return a;
+    const float c0 = fmaxf((float)(s0.x + s0.y), 0.f), c1 = fmaxf((float)(s1.x + s1.y), 0.f),
+                c2 = fmaxf((float)(s2.x + s2.y), 0.f);
+    if (j.integrator == XT_INTEGRATOR_STENCIL || j.integrator == XT_INTEGRATOR_WIREFRAME) {
+        const float rgb = c0 > 0.f ? 1.f : 0.f;
+        return make_float4(rgb, rgb, rgb, fminf(c0, 1.f));
+    }
+    return make_float4(c0, c1, c2, 1.f);
+}
+
+// A lane's totals, written to pinned host memory by its last kernel.
+struct JobTotals {
+    unsigned long long queries, retests, steps_exceeded, trace_fail;
+};
+
 // Per pixel of tile positions [q0, q0 + qn), samples of this pass in sample
 // order (radiance of sample pass_base + sl at rad[sl * qn + q - q0]).
 // REFERENCE reproduces the float read-modify-write of each integrator
 // (tile_t::read/write, lib/nimg/color.cc:35-40 clamps); FP64 keeps a
-// Neumaier sum per channel.
+// Neumaier sum per channel. The first pass starts from zero sums instead of
+// reading them; with `out`, the last pass writes the image instead of the sums:
+// a job of one pass (64 bytes of sums a pixel) touches neither.
 static __global__ __launch_bounds__(XT_BLOCK) void k_accumulate(const JobDev j, uint32_t pass_base, uint32_t spp_pass,
                                                          uint32_t q0, uint32_t qn, const float4 *rad,
-                                                         const double *nrm64, float4 *accf, double2 *acc64) {
+                                                         const double *nrm64, float4 *accf, double2 *acc64, bool first,
+                                                         float4 *out, const Counters *cnt, JobTotals *totals) {
     const uint32_t stride = gridDim.x * blockDim.x;
+    if (totals && blockIdx.x == 0 && threadIdx.x == 0)
+        *totals = JobTotals{cnt->queries, cnt->retests, cnt->steps_exceeded, cnt->trace_fail};
     for (uint32_t qi = blockIdx.x * blockDim.x + threadIdx.x; qi < qn; qi += stride) {
         const uint32_t q = q0 + qi;
         uint32_t x, y;
         if (!slot_pixel(j, q, x, y)) continue;
         const uint32_t pix = y * j.W + x;
-        float4 a = accf[pix];
-        double2 s0 = acc64[3 * (size_t)pix], s1 = acc64[3 * (size_t)pix + 1], s2 = acc64[3 * (size_t)pix + 2];
+        float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+        double2 s0 = make_double2(0.0, 0.0), s1 = s0, s2 = s0;
+        if (!first) {
+            a = accf[pix];
+            s0 = acc64[3 * (size_t)pix];
+            s1 = acc64[3 * (size_t)pix + 1];
+            s2 = acc64[3 * (size_t)pix + 2];
+        }
         for (uint32_t sl = 0; sl < spp_pass; ++sl) {
             if (pass_base + sl >= j.total) break;
             const float4 v = rad[sl * qn + qi];
@@ -1275,6 +1315,10 @@ static __global__ __launch_bounds__(XT_BLOCK) void k_accumulate(const JobDev j, 
                 neumaier_add(s2, xs[2]);
             }
         }
+        if (out) {
+            out[pix] = resolve_px(j, a, s0, s1, s2);
+            continue;
+        }
         accf[pix] = a;
         acc64[3 * (size_t)pix] = s0;
         acc64[3 * (size_t)pix + 1] = s1;
@@ -1286,24 +1330,8 @@ static __global__ __launch_bounds__(XT_BLOCK) void k_resolve(const JobDev j, con
                                                       float4 *out) {
     const uint32_t n = j.W * j.H;
     const uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += stride) {
-        if (j.accum == XT_ACCUM_REFERENCE) {
-            out[p] = accf[p];
-            continue;
-        }
-        float c[3];
-        for (int k = 0; k < 3; ++k) {
-            const double2 s = acc64[3 * (size_t)p + k];
-            c[k] = fmaxf((float)(s.x + s.y), 0.f);
-        }
-        if (j.integrator == XT_INTEGRATOR_STENCIL || j.integrator == XT_INTEGRATOR_WIREFRAME) {
-            const float a = fminf(c[0], 1.f);
-            const float rgb = c[0] > 0.f ? 1.f : 0.f;
-            out[p] = make_float4(rgb, rgb, rgb, a);
-        } else {
-            out[p] = make_float4(c[0], c[1], c[2], 1.f);
-        }
-    }
+    for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += stride)
+        out[p] = resolve_px(j, accf[p], acc64[3 * (size_t)p], acc64[3 * (size_t)p + 1], acc64[3 * (size_t)p + 2]);
 }
 
 #pragma clang fp contract(off)

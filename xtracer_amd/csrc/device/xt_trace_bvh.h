@@ -64,12 +64,13 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 template <int STACK, int BS>
 static __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(XT_W_WAVES))) void k_trace_bvh(
     const SceneView S, const Queue in, const uint32_t *in_count, float4 *hit, uint32_t *retest_list,
-    uint4 *recheck_list, Counters *cnt, uint32_t nseg) {
+    uint4 *recheck_list, const TraceCtl T) {
+    Counters *const cnt = T.cnt;
     __shared__ uint32_t wstk[STACK * BS];
     __shared__ uint4 wbuf[BS / 64][64 * 8];
     uint32_t *const stk = wstk + threadIdx.x;
     const uint32_t n = *in_count;
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&cnt->queries, (unsigned long long)n);
+    trace_open(T, n);
     const uint32_t lane = lane_id();
     const uint32_t waves = gridDim.x * (BS / 64);
     const uint32_t wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -77,7 +78,7 @@ static __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(XT_W_
     uint4 *const buf = wbuf[wid];
     const float4 *const recs = S.kd_indexed ? S.prims : S.bvh_leaf;
     RaySource R;
-    source_init(R, n, waves, nseg);
+    source_init(R, n, waves, T);
     bool more = true;
     const float smax = fmaxf(fmaxf(fmaxf(fabsf(S.kb_lo[0]), fabsf(S.kb_hi[0])),
                                    fmaxf(fabsf(S.kb_lo[1]), fabsf(S.kb_hi[1]))),
@@ -102,9 +103,9 @@ static __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(XT_W_
                     finish_ray(S, in, hit, cnt, ri, o, origin, true, best, recs, best_rec, mark, full);
                 if (__builtin_amdgcn_ballot_w64(mark)) {
                     const bool rf = mark && full, rc = mark && !full;
-                    const uint32_t slot = wave_append(rf, &cnt->n[CNT_RETEST]);
+                    const uint32_t slot = wave_append(rf, &cnt->n[CNT_RETEST + T.par]);
                     if (rf) retest_list[slot] = ri;
-                    const uint32_t cslot = wave_append(rc, &cnt->n[CNT_RECHECK]);
+                    const uint32_t cslot = wave_append(rc, &cnt->n[CNT_RECHECK + T.par]);
                     if (rc) recheck_list[cslot] = make_uint4(ri, best.c0, best.c1, XT_NONE);
                 }
                 done = false;

@@ -21,17 +21,18 @@
 template <int STACK, int BS>
 static __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(XT_KD_WAVES))) void k_trace_kd(
     const SceneView S, const Queue in, const uint32_t *in_count, float4 *hit, uint32_t *retest_list,
-    uint4 *recheck_list, Counters *cnt, uint32_t nseg) {
+    uint4 *recheck_list, const TraceCtl T) {
+    Counters *const cnt = T.cnt;
     constexpr uint32_t SLOTS = STACK + 1;
     __shared__ uint2 kstk[SLOTS * BS];
     uint2 *const stk = kstk + threadIdx.x;
     const uint32_t n = *in_count;
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&cnt->queries, (unsigned long long)n);
+    trace_open(T, n);
     const uint32_t lane = lane_id();
     const uint32_t waves = gridDim.x * (BS / 64);
     const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (BS / 64) + (threadIdx.x >> 6));
     RaySource R;
-    source_init(R, n, waves, nseg);
+    source_init(R, n, waves, T);
     bool more = true;
 
     const XtKdNode root = S.kd[0];
@@ -55,9 +56,9 @@ static __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(XT_KD
                 if (done) finish_ray(S, in, hit, cnt, ri, o, origin, ok, best, S.prims, best.prim, mark, full);
                 const bool rf = mark && full, rc = mark && !full;
                 if (__builtin_amdgcn_ballot_w64(mark)) {
-                    const uint32_t slot = wave_append(rf, &cnt->n[CNT_RETEST]);
+                    const uint32_t slot = wave_append(rf, &cnt->n[CNT_RETEST + T.par]);
                     if (rf) retest_list[slot] = ri;
-                    const uint32_t cslot = wave_append(rc, &cnt->n[CNT_RECHECK]);
+                    const uint32_t cslot = wave_append(rc, &cnt->n[CNT_RECHECK + T.par]);
                     if (rc) recheck_list[cslot] = make_uint4(ri, best.c0, best.c1, XT_NONE);
                 }
                 done = false;

@@ -20,15 +20,17 @@
 // runs of up to 512 rays leave 0.1 ms; a queue that one run per wave covers
 // needs no atomic at all (100,003 rays: 219 to 120 us).
 struct RaySource {
-    uint32_t n, base, sh, len, xcd;  // rays, first dealt ray, log2 of a stretch (or, sh = 32, its length)
+    uint32_t n, base, sh, len, par, xcd;  // rays, first dealt ray, log2 of a stretch (or, sh = 32, its length)
     uint32_t waves;                  // per XCD
     uint32_t cur, end;               // the run in hand: rays (first run), or positions on the XCD's stretches
     uint32_t seen;                   // the XCD's cursor when last seen
     uint32_t state;                  // 0: before the first run, 1: in it, 2: dealt runs
 };
 
-__device__ __forceinline__ void source_init(RaySource &R, uint32_t n, uint32_t waves, uint32_t nseg) {
+__device__ __forceinline__ void source_init(RaySource &R, uint32_t n, uint32_t waves, const TraceCtl &T) {
+    const uint32_t nseg = T.nseg;
     R.n = n;
+    R.par = T.par;
     R.base = waves * 64u < n ? waves * 64u : n;
     R.sh = nseg == 1u ? (uint32_t)XT_STRETCH_LOG : 32u;
     R.len = nseg == 1u ? 1u << XT_STRETCH_LOG : ((n - R.base) / 8u + 64u) & ~63u;
@@ -69,7 +71,7 @@ __device__ __forceinline__ bool source_next(RaySource &R, Counters *cnt, uint32_
             uint32_t want = (total - R.seen) / (2u * R.waves) & ~63u;
             want = want < 64u ? 64u : (want > XT_RUN_MAX ? XT_RUN_MAX : want);
             uint32_t c = 0;
-            if (lane == 0) c = atomicAdd(&cnt->xcd[R.xcd * XT_CURSOR_STRIDE], want);
+            if (lane == 0) c = atomicAdd(&cnt->cursor[R.par][R.xcd * XT_CURSOR_STRIDE], want);
             c = __builtin_amdgcn_readfirstlane(c);
             R.seen = c + want;
             if (c < total) {
@@ -83,7 +85,7 @@ __device__ __forceinline__ bool source_next(RaySource &R, Counters *cnt, uint32_
         uint32_t at = 0;
         const uint32_t x = (R.xcd + 1u + lane) & 7u;
         if (lane < 8u) {
-            at = __hip_atomic_load(&cnt->xcd[x * XT_CURSOR_STRIDE], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            at = __hip_atomic_load(&cnt->cursor[R.par][x * XT_CURSOR_STRIDE], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             left = at < source_count(R, x);
         }
         const unsigned long long m = __builtin_amdgcn_ballot_w64(left);

@@ -10,7 +10,7 @@
 
 #include "device/xt_kernels.h"
 
-#define XT_TRACE_EVENTS 512
+#define XT_TRACE_STAMPS 256
 
 struct DevScene {
     SceneView view;
@@ -57,6 +57,13 @@ struct AccumBuffers {
     uint64_t bytes = 0;
 };
 
+// What kernels report to the host without a copy: fine-grained pinned memory.
+struct HostReports {
+    uint64_t stamp[2 * XT_TRACE_STAMPS];  // wall clock at a timed trace launch's start and end
+    uint32_t count[XT_MAX_LANES];         // queue counts of the early-stop check
+    JobTotals totals[XT_MAX_LANES];
+};
+
 struct ServeState;  // continuous-batching server (xt_serve.hip)
 
 struct xt_dev {
@@ -71,13 +78,11 @@ struct xt_dev {
     WaveBuffers wave;
     AccumBuffers accum;
     Counters *host_counters = nullptr;  // pinned, XT_MAX_LANES blocks
+    HostReports *reports = nullptr;     // pinned, written by kernels (xt_ensure_reports)
+    double clock_khz = 100000.0;        // of the stamps
     uint64_t *host_words = nullptr;     // pinned, 8 KiB: read-backs of an index build
-    uint32_t *host_snap = nullptr;      // pinned, 2 x XT_MAX_LANES queue counts of the early-stop check
-    hipEvent_t snap_ev[2][XT_MAX_LANES] = {};
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    hipEvent_t tev[XT_TRACE_EVENTS];
-    int trace_launches = 0;
-    std::vector<int> timed_pairs;
+    int trace_launches = 0;  // trace launches with a stamp in this call
     ServeState *serve = nullptr;
     xt_tuning tuning{12, 256, 64u << 20, 0, 1, 1, 1, 1, 2};
     void *scratch = nullptr;  // this device's address of xt_trace_device_static's scratch array
@@ -105,7 +110,12 @@ struct WaveLane {
     Counters *cnt = nullptr;
 };
 int xt_launch_trace(xt_dev *d, const DevScene &ds, int accel, int qi, const WaveLane &lane, const double *ray64,
-                    uint32_t *flags, bool time_it, hipStream_t st);
+                    uint32_t *flags, bool time_it, hipStream_t st, uint32_t *post = nullptr);
+int xt_ensure_reports(xt_dev *d);
+// Milliseconds between two stamps.
+inline double xt_stamp_ms(const xt_dev *d, uint64_t a, uint64_t b) {
+    return b > a ? (double)(b - a) / d->clock_khz : 0.0;
+}
 // The buffers one trace launch reads and writes.
 struct TraceBufs {
     Queue q;
@@ -115,6 +125,8 @@ struct TraceBufs {
     uint4 *recheck = nullptr;
     Counters *cnt = nullptr;
     size_t cap = 0;  // queue capacity (sizes the grids)
+    uint32_t par = 0;          // parity of the round (Counters)
+    uint32_t *post = nullptr;  // pinned: where the trace posts its ray count
 };
 int xt_launch_trace_bufs(xt_dev *d, const DevScene &ds, int accel, const TraceBufs &B, const double *ray64,
                          uint32_t *flags, bool time_it, hipStream_t st);

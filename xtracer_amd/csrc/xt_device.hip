@@ -163,11 +163,11 @@ extern "C" {
 // a device address: xt_dev_create looks its address up per device.
 struct StaticTraceScratch {
     Counters cnt;
-    uint32_t pad[512 - sizeof(Counters) / 4];
+    uint32_t pad[1024 - sizeof(Counters) / 4];
     uint4 recheck[XT_TRACE_STATIC_MAX_RAYS];
     uint32_t retest[XT_TRACE_STATIC_MAX_RAYS];
 };
-static_assert(sizeof(Counters) % 4 == 0 && sizeof(Counters) < 2048, "scratch header");
+static_assert(sizeof(Counters) % 4 == 0 && sizeof(Counters) < 4096, "scratch header");
 __device__ __align__(256) StaticTraceScratch scratch;
 
 int xt_dev_create(xt_dev **out, int hip_device, uint64_t hbm_budget_bytes) {
@@ -185,7 +185,9 @@ int xt_dev_create(xt_dev **out, int hip_device, uint64_t hbm_budget_bytes) {
     }
     hipEventCreate(&d->ev0);
     hipEventCreate(&d->ev1);
-    for (int i = 0; i < XT_TRACE_EVENTS; ++i) hipEventCreate(&d->tev[i]);
+    int khz = 0;
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, hip_device) == hipSuccess && khz > 0)
+        d->clock_khz = khz;
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, hip_device) == hipSuccess) {
         d->n_cu = prop.multiProcessorCount;
@@ -209,11 +211,8 @@ void xt_dev_destroy(xt_dev *d) {
     xt_dev_free_wave(d);
     xt_dev_free_accum(d);
     if (d->host_counters) hipHostFree(d->host_counters);
-    if (d->host_snap) hipHostFree(d->host_snap);
+    if (d->reports) hipHostFree(d->reports);
     if (d->host_words) hipHostFree(d->host_words);
-    for (auto &row : d->snap_ev)
-        for (hipEvent_t e : row)
-            if (e) hipEventDestroy(e);
     for (int k = 0; k < XT_LANE_STREAMS; ++k) {
         if (d->lane_stream[k]) hipStreamDestroy(d->lane_stream[k]);
         if (d->lane_ev[k]) hipEventDestroy(d->lane_ev[k]);
@@ -221,7 +220,6 @@ void xt_dev_destroy(xt_dev *d) {
     if (d->fork_ev) hipEventDestroy(d->fork_ev);
     hipEventDestroy(d->ev0);
     hipEventDestroy(d->ev1);
-    for (int i = 0; i < XT_TRACE_EVENTS; ++i) hipEventDestroy(d->tev[i]);
     hipStreamDestroy(d->stream);
     delete d;
 }
@@ -464,7 +462,7 @@ int xt_scene_release(xt_dev *d, uint32_t scene_id) {
 // blocks the CU keeps resident, from the occupancy calculator.
 template <int STACK, int BS>
 static void launch_kd_trace_sb(unsigned per_cu, int n_cu, size_t cap, hipStream_t st, const SceneView &v,
-                               const Queue &q, const uint32_t *count, float4 *hit, uint32_t *retest, uint4 *recheck, Counters *cnt, uint32_t nseg) {
+                               const Queue &q, const uint32_t *count, float4 *hit, uint32_t *retest, uint4 *recheck, const TraceCtl &T) {
     static int resident = 0;
     if (per_cu == 0) {
         if (resident == 0) {
@@ -479,14 +477,13 @@ static void launch_kd_trace_sb(unsigned per_cu, int n_cu, size_t cap, hipStream_
     }
     const size_t need = (cap + BS - 1) / BS;
     const unsigned g = (unsigned)std::max<size_t>(1, std::min<size_t>(need, (size_t)n_cu * per_cu));
-    hipLaunchKernelGGL((k_trace_kd<STACK, BS>), dim3(g), dim3(BS), 0, st, v, q, count, hit, retest, recheck,
-                       cnt, nseg);
+    hipLaunchKernelGGL((k_trace_kd<STACK, BS>), dim3(g), dim3(BS), 0, st, v, q, count, hit, retest, recheck, T);
 }
 
 template <int STACK, int BS>
 static void launch_bvh_trace_sb(unsigned per_cu, int n_cu, size_t cap, hipStream_t st, const SceneView &v,
                                 const Queue &q, const uint32_t *count, float4 *hit, uint32_t *retest, uint4 *recheck,
-                                Counters *cnt, uint32_t nseg) {
+                                const TraceCtl &T) {
     static int resident = 0;
     if (per_cu == 0) {
         if (resident == 0) {
@@ -499,78 +496,86 @@ static void launch_bvh_trace_sb(unsigned per_cu, int n_cu, size_t cap, hipStream
     }
     const size_t need = (cap + BS - 1) / BS;
     const unsigned g = (unsigned)std::max<size_t>(1, std::min<size_t>(need, (size_t)n_cu * per_cu));
-    hipLaunchKernelGGL((k_trace_bvh<STACK, BS>), dim3(g), dim3(BS), 0, st, v, q, count, hit, retest, recheck, cnt, nseg);
+    hipLaunchKernelGGL((k_trace_bvh<STACK, BS>), dim3(g), dim3(BS), 0, st, v, q, count, hit, retest, recheck, T);
 }
 
 template <int STACK>
 static void launch_bvh_trace_s(unsigned bs, unsigned per_cu, int n_cu, size_t cap, hipStream_t st, const SceneView &v,
                                const Queue &q, const uint32_t *count, float4 *hit, uint32_t *retest, uint4 *recheck,
-                               Counters *cnt, uint32_t nseg) {
-    if (bs == 128) launch_bvh_trace_sb<STACK, 128>(per_cu, n_cu, cap, st, v, q, count, hit, retest, recheck, cnt, nseg);
-    else launch_bvh_trace_sb<STACK, 256>(per_cu, n_cu, cap, st, v, q, count, hit, retest, recheck, cnt, nseg);
+                               const TraceCtl &T) {
+    if (bs == 128) launch_bvh_trace_sb<STACK, 128>(per_cu, n_cu, cap, st, v, q, count, hit, retest, recheck, T);
+    else launch_bvh_trace_sb<STACK, 256>(per_cu, n_cu, cap, st, v, q, count, hit, retest, recheck, T);
 }
 
 template <int STACK>
 static void launch_kd_trace_s(unsigned bs, unsigned per_cu, int n_cu, size_t cap, hipStream_t st, const SceneView &v,
-                              const Queue &q, const uint32_t *count, float4 *hit, uint32_t *retest, uint4 *recheck, Counters *cnt, uint32_t nseg) {
-    if (bs == 128) launch_kd_trace_sb<STACK, 128>(per_cu, n_cu, cap, st, v, q, count, hit, retest, recheck, cnt, nseg);
-    else launch_kd_trace_sb<STACK, 256>(per_cu, n_cu, cap, st, v, q, count, hit, retest, recheck, cnt, nseg);
+                              const Queue &q, const uint32_t *count, float4 *hit, uint32_t *retest, uint4 *recheck, const TraceCtl &T) {
+    if (bs == 128) launch_kd_trace_sb<STACK, 128>(per_cu, n_cu, cap, st, v, q, count, hit, retest, recheck, T);
+    else launch_kd_trace_sb<STACK, 256>(per_cu, n_cu, cap, st, v, q, count, hit, retest, recheck, T);
 }
 
 static void launch_kd_trace(const xt_tuning &tn, uint32_t bvh_depth, int n_cu, size_t cap, hipStream_t st, const SceneView &view,
-                            const Queue &q, const uint32_t *count, float4 *hit, uint32_t *retest, uint4 *recheck, Counters *cnt) {
-    const uint32_t nseg = tn.trace_segments == XT_TRACE_SEGMENTS ? XT_TRACE_SEGMENTS : 1u;
+                            const Queue &q, const uint32_t *count, float4 *hit, uint32_t *retest, uint4 *recheck, const TraceCtl &T) {
     SceneView v = view;
     v.kd_indexed = tn.kd_leaf == 2;
     const unsigned bs = tn.trace_block, pc = tn.trace_blocks_per_cu;
     if (v.bvh) {
         // a walk holds a group for each level but the root's and the leaves'
         const uint32_t s = bvh_depth < 2 ? 0 : bvh_depth - 2;
-        if (s <= 8) launch_bvh_trace_s<8>(bs, pc, n_cu, cap, st, v, q, count, hit, retest, recheck, cnt, nseg);
-        else if (s <= 12) launch_bvh_trace_s<12>(bs, pc, n_cu, cap, st, v, q, count, hit, retest, recheck, cnt, nseg);
-        else launch_bvh_trace_sb<24, 128>(pc, n_cu, cap, st, v, q, count, hit, retest, recheck, cnt, nseg);
+        if (s <= 8) launch_bvh_trace_s<8>(bs, pc, n_cu, cap, st, v, q, count, hit, retest, recheck, T);
+        else if (s <= 12) launch_bvh_trace_s<12>(bs, pc, n_cu, cap, st, v, q, count, hit, retest, recheck, T);
+        else launch_bvh_trace_sb<24, 128>(pc, n_cu, cap, st, v, q, count, hit, retest, recheck, T);
         return;
     }
     switch (tn.kd_stack) {
-        case 8: launch_kd_trace_s<8>(bs, pc, n_cu, cap, st, v, q, count, hit, retest, recheck, cnt, nseg); break;
-        case 12: launch_kd_trace_s<12>(bs, pc, n_cu, cap, st, v, q, count, hit, retest, recheck, cnt, nseg); break;
-        case 24: launch_kd_trace_s<24>(bs, pc, n_cu, cap, st, v, q, count, hit, retest, recheck, cnt, nseg); break;
-        default: launch_kd_trace_s<16>(bs, pc, n_cu, cap, st, v, q, count, hit, retest, recheck, cnt, nseg); break;
+        case 8: launch_kd_trace_s<8>(bs, pc, n_cu, cap, st, v, q, count, hit, retest, recheck, T); break;
+        case 12: launch_kd_trace_s<12>(bs, pc, n_cu, cap, st, v, q, count, hit, retest, recheck, T); break;
+        case 24: launch_kd_trace_s<24>(bs, pc, n_cu, cap, st, v, q, count, hit, retest, recheck, T); break;
+        default: launch_kd_trace_s<16>(bs, pc, n_cu, cap, st, v, q, count, hit, retest, recheck, T); break;
     }
 }
 
 // Launches trace + FP64 re-check / re-test over queue `q` (count at `count`)
 // into explicit buffers.
+int xt_ensure_reports(xt_dev *d) {
+    if (!d->reports)
+        XT_TRY(hipHostMalloc((void **)&d->reports, sizeof(HostReports), hipHostMallocCoherent | hipHostMallocMapped));
+    return XT_OK;
+}
+
+// A trace launch and the FP64 kernel behind it. A timed launch's start and end
+// are the wall clock when its first workgroup starts and when the first one
+// behind it does: two events around it cost 12 us.
 int xt_launch_trace_bufs(xt_dev *d, const DevScene &ds, int accel, const TraceBufs &B, const double *ray64,
                          uint32_t *flags, bool time_it, hipStream_t st) {
-    const bool timed = time_it && d->trace_launches < XT_TRACE_EVENTS - 1;
-    if (timed) hipEventRecord(d->tev[d->trace_launches], st);
     const xt_tuning &tn = d->tuning;
+    TraceCtl T;
+    T.cnt = B.cnt;
+    T.par = B.par;
+    T.nseg = tn.trace_segments == XT_TRACE_SEGMENTS ? XT_TRACE_SEGMENTS : 1u;
+    T.stamp = nullptr;
+    T.post = B.post;
+    if (time_it && d->trace_launches < XT_TRACE_STAMPS) {
+        const int rc = xt_ensure_reports(d);
+        if (rc) return rc;
+        T.stamp = d->reports->stamp + 2 * d->trace_launches++;
+    }
     if (accel == XT_ACCEL_OCTREE) {
         // 16 resident 64-lane blocks per CU (LDS: 20 KB each)
         const unsigned g = (unsigned)std::min<size_t>(B.cap / XT_OCT_BLOCK + 1, (size_t)d->n_cu * 16);
         hipLaunchKernelGGL(k_trace_oct, dim3(g), dim3(XT_OCT_BLOCK), 0, st,
-                           ds.view, B.q, B.count, B.hit, B.retest, B.recheck, B.cnt,
-                           tn.trace_segments == XT_TRACE_SEGMENTS ? XT_TRACE_SEGMENTS : 1u);
+                           ds.view, B.q, B.count, B.hit, B.retest, B.recheck, T);
     } else {
-        launch_kd_trace(tn, ds.bvh_depth, d->n_cu, B.cap, st, ds.view, B.q, B.count, B.hit, B.retest, B.recheck, B.cnt);
-    }
-    if (timed) {
-        hipEventRecord(d->tev[d->trace_launches + 1], st);
-        d->timed_pairs.push_back(d->trace_launches);
-        d->trace_launches += 2;
+        launch_kd_trace(tn, ds.bvh_depth, d->n_cu, B.cap, st, ds.view, B.q, B.count, B.hit, B.retest, B.recheck, T);
     }
     XT_LAUNCHED();
-    hipLaunchKernelGGL(k_recheck, dim3(grid_for(B.cap / 64 + 1, XT_BLOCK, 256)), dim3(XT_BLOCK), 0, st,
-                       ds.view, B.q, B.hit, B.recheck, B.retest, B.cnt, ray64, flags);
-    XT_LAUNCHED();
-    if (accel == XT_ACCEL_OCTREE) {
-        hipLaunchKernelGGL(k_retest<XT_ACCEL_OCTREE>, dim3(grid_for(B.cap / 64 + 1, XT_OCT_BLOCK, 2048)),
-                           dim3(XT_OCT_BLOCK), 0, st, ds.view, B.q, B.hit, B.retest, B.cnt, ray64, flags);
-    } else {
-        hipLaunchKernelGGL(k_retest<XT_ACCEL_KDTREE>, dim3(grid_for(B.cap / 64 + 1, XT_BLOCK, 1024)), dim3(XT_BLOCK),
-                           0, st, ds.view, B.q, B.hit, B.retest, B.cnt, ray64, flags);
-    }
+    const dim3 rg(grid_for(B.cap / 64 + 1, XT_RECHECK_BLOCK, 2048)), rb(XT_RECHECK_BLOCK);
+    if (accel == XT_ACCEL_OCTREE)
+        hipLaunchKernelGGL(k_recheck<XT_ACCEL_OCTREE>, rg, rb, 0, st, ds.view, B.q, B.hit, B.recheck, B.retest, T, ray64,
+                           flags);
+    else
+        hipLaunchKernelGGL(k_recheck<XT_ACCEL_KDTREE>, rg, rb, 0, st, ds.view, B.q, B.hit, B.recheck, B.retest, T, ray64,
+                           flags);
     XT_LAUNCHED();
     return XT_OK;
 }
@@ -578,7 +583,7 @@ int xt_launch_trace_bufs(xt_dev *d, const DevScene &ds, int accel, const TraceBu
 // Launches trace + FP64 re-test over queue `qi` of a lane (count in
 // lane.cnt->n[qi]).
 int xt_launch_trace(xt_dev *d, const DevScene &ds, int accel, int qi, const WaveLane &L, const double *ray64,
-                    uint32_t *flags, bool time_it, hipStream_t st) {
+                    uint32_t *flags, bool time_it, hipStream_t st, uint32_t *post) {
     WaveBuffers &w = d->wave;
     TraceBufs B;
     B.q = Queue{w.q[qi].r0 + L.off, w.q[qi].r1 + L.off, w.q[qi].path + L.off};
@@ -588,6 +593,8 @@ int xt_launch_trace(xt_dev *d, const DevScene &ds, int accel, int qi, const Wave
     B.recheck = w.recheck + L.off;
     B.cnt = L.cnt;
     B.cap = L.cap;
+    B.par = (uint32_t)qi;
+    B.post = post;
     return xt_launch_trace_bufs(d, ds, accel, B, ray64, flags, time_it, st);
 }
 
@@ -607,24 +614,17 @@ extern "C" int xt_trace_device(xt_dev *d, uint32_t scene_id, int accel, const vo
     w.q[0].r0 = (float4 *)ray0;
     w.q[0].r1 = (float4 *)ray1;
     w.hit = (float4 *)hit;
-    hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, d->stream, w.cnt, 0x800000ffu);
-    // paths are only read by the FP64 re-test when FP64 rays are given; set
-    // the count with a one-thread kernel instead of a memset (graph-safe)
-    hipLaunchKernelGGL(k_set_count, dim3(1), dim3(1), 0, d->stream, w.cnt, 0u, (uint32_t)n);
+    // paths are only read by the FP64 re-test when FP64 rays are given
+    hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, d->stream, w.cnt, (uint32_t)n);
     if (flags) hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(n, 256, 4096)), dim3(256), 0, d->stream, flags, 0u, (size_t)n);
     d->trace_launches = 0;
-    d->timed_pairs.clear();
     rc = xt_launch_trace(d, it->second, accel, 0, WaveLane{0, (size_t)n, w.cnt}, nullptr, flags, kernel_ms != nullptr, d->stream);
     w.q[0].r0 = save0;
     w.q[0].r1 = save1;
     w.hit = saveh;
     if (rc) return rc;
     XT_TRY(hipStreamSynchronize(d->stream));
-    if (kernel_ms && !d->timed_pairs.empty()) {
-        float ms = 0.f;
-        hipEventElapsedTime(&ms, d->tev[d->timed_pairs[0]], d->tev[d->timed_pairs[0] + 1]);
-        *kernel_ms = ms;
-    }
+    if (kernel_ms) *kernel_ms = (float)xt_stamp_ms(d, d->reports->stamp[0], d->reports->stamp[1]);
     return XT_OK;
 }
 
@@ -647,8 +647,7 @@ extern "C" int xt_trace_device_static(xt_dev *d, uint32_t scene_id, int accel, c
     }
     XT_TRY(hipSetDevice(d->device));
     StaticTraceScratch *sc = (StaticTraceScratch *)d->scratch;
-    hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, d->stream, &sc->cnt, 0x800000ffu);
-    hipLaunchKernelGGL(k_set_count, dim3(1), dim3(1), 0, d->stream, &sc->cnt, 0u, (uint32_t)n);
+    hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, d->stream, &sc->cnt, (uint32_t)n);
     if (flags) hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(n, 256, 4096)), dim3(256), 0, d->stream, flags, 0u, (size_t)n);
     XT_LAUNCHED();
     TraceBufs B;
@@ -734,11 +733,9 @@ extern "C" int xt_trace(xt_dev *d, uint32_t scene_id, int accel, const xt_rays *
     Queue q{w.q[0].r0, w.q[0].r1, w.q[0].path};
     hipLaunchKernelGGL(k_pack_rays, dim3(grid_for(n, 256, 4096)), dim3(256), 0, d->stream, soa[0], soa[1], soa[2],
                        soa[3], soa[4], soa[5], q, (uint32_t)n);
-    hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, d->stream, w.cnt, 0x800000ffu);
-    hipLaunchKernelGGL(k_set_count, dim3(1), dim3(1), 0, d->stream, w.cnt, 0u, (uint32_t)n);
+    hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, d->stream, w.cnt, (uint32_t)n);
     hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(n, 256, 4096)), dim3(256), 0, d->stream, w.flags, 0u, (size_t)n);
     d->trace_launches = 0;
-    d->timed_pairs.clear();
     rc = xt_launch_trace(d, it->second, accel, 0, WaveLane{0, (size_t)n, w.cnt}, nullptr, w.flags, false, d->stream);
     if (rc) return rc;
     hipLaunchKernelGGL(k_unpack_hits, dim3(grid_for(n, 256, 4096)), dim3(256), 0, d->stream, w.hit, soa[0],

@@ -32,8 +32,12 @@
         }                                                                             \
     } while (0)
 
-namespace {
-}  // namespace
+// Paths of a pass from which frame_lanes 2 cuts it into two groups. The second
+// group costs launches, a fork and a join, and hides one group's launch tails
+// behind the other's work: 1001x701 normals (0.70 M paths) take 614 us in two
+// groups and 710 in one, 256x256x4 paths (0.26 M) 764 and 759, a 33x17 frame
+// 70 and 44.
+#define XT_TWO_GROUPS (1u << 19)
 
 int xt_job_check(xt_dev *d, const xt_job *job, JobDev &j, const DevScene **ds_out) {
     if (!job) return XT_E_INVALID;
@@ -200,11 +204,10 @@ int xt_ensure_host_counters(xt_dev *d) {
 // 0 holding the camera rays. With several groups, each group's kernels run
 // on a stream of its own so that one group's launch tails overlap another's
 // work; the device stream forks to them and joins them again at the end.
-// Every second round past the second, each live group's next queue count is
-// copied to pinned memory on the group's stream. The host then reads the
-// copies of the check before, two rounds back, so that the device still has
-// two rounds queued while the host waits and the groups never wait for each
-// other, and issues no more rounds to groups whose paths have all ended.
+// Every second round's trace posts its ray count to host memory, and the host
+// reads it once the next round is queued: no more rounds are issued to groups
+// whose paths have all ended, and the device has a round and a half queued while
+// the host waits.
 int xt_run_rounds(xt_dev *d, PassGroup *groups, int n_groups, bool time_trace, const GroupHook *before,
                   const GroupHook *after) {
     WaveBuffers &w = d->wave;
@@ -225,11 +228,9 @@ int xt_run_rounds(xt_dev *d, PassGroup *groups, int n_groups, bool time_trace, c
         }
     }
     if (n_st && !d->fork_ev) XT_TRY(hipEventCreateWithFlags(&d->fork_ev, hipEventDisableTiming));
-    if (!d->host_snap)
-        XT_TRY(hipHostMalloc((void **)&d->host_snap, 2 * XT_MAX_LANES * sizeof(uint32_t), hipHostMallocDefault));
-    for (int s = 0; s < 2; ++s)
-        for (int k = 0; k < n_groups; ++k)
-            if (!d->snap_ev[s][k]) XT_TRY(hipEventCreateWithFlags(&d->snap_ev[s][k], hipEventDisableTiming));
+    int rc0 = xt_ensure_reports(d);
+    if (rc0) return rc0;
+    HostReports &H = *d->reports;
     auto stream_of = [&](int k) { return n_st ? d->lane_stream[k % n_st] : d->stream; };
     if (n_st) {
         XT_TRY(hipEventRecord(d->fork_ev, d->stream));
@@ -253,44 +254,52 @@ int xt_run_rounds(xt_dev *d, PassGroup *groups, int n_groups, bool time_trace, c
         const int rc = (*before)(k, stream_of(k));
         if (rc) return rc;
     }
-    int qi = 0, slot = 0;
-    bool pending = false;
+    // the count that group k's trace posted, or an error of its stream
+    auto posted = [&](int k, uint32_t &n) -> int {
+        for (uint32_t spin = 1;; ++spin) {
+            n = __atomic_load_n(&H.count[k], __ATOMIC_RELAXED);
+            if (n != XT_NONE) return XT_OK;
+            if (spin % 4096u) continue;
+            const hipError_t e = hipStreamQuery(stream_of(k));
+            if (e == hipErrorNotReady) continue;
+            XT_TRY(e);
+            n = __atomic_load_n(&H.count[k], __ATOMIC_RELAXED);
+            return XT_OK;
+        }
+    };
+    int qi = 0;
     for (uint32_t r = 0; r < max_rounds; ++r) {
         for (int k = 0; k < n_groups; ++k) {
             PassGroup &G = groups[k];
             if (!G.live || r >= G.rounds) continue;
             const hipStream_t st = stream_of(k);
-            hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, st, G.lane.cnt,
-                               (1u << (qi ^ 1)) | (1u << CNT_RETEST) | (1u << CNT_CURSOR) | (1u << CNT_RECHECK));
+            uint32_t *post = nullptr;
+            if (r >= 2 && r % 2 == 0 && r + 2 < G.rounds) {  // read below, one round later
+                post = &H.count[k];
+                __atomic_store_n(post, XT_NONE, __ATOMIC_RELAXED);
+            }
             const bool fp64_rays = xt_needs_ray64(G.integrator) && r == 0;
             int rc = xt_launch_trace(d, *G.ds, (int)G.accel, qi, G.lane, fp64_rays ? w.ray64 : nullptr, nullptr,
-                                     time_trace, st);
+                                     time_trace, st, post);
             if (rc) return rc;
             rc = xt_launch_shade(d, *G.ds, G.integrator, r, qi, G.lane, st);
             if (rc) return rc;
         }
         qi ^= 1;
-        if (max_rounds > 2 && r + 1 < max_rounds && (r % 2 == 1)) {
-            if (pending) {  // the previous check: paths left after round r - 2
-                bool any = false;
-                for (int k = 0; k < n_groups; ++k) {
-                    PassGroup &G = groups[k];
-                    if (!G.live) continue;
-                    XT_TRY(hipEventSynchronize(d->snap_ev[slot ^ 1][k]));
-                    if (r + 1 >= G.rounds || d->host_snap[(slot ^ 1) * XT_MAX_LANES + k] == 0) G.live = false;
-                    any = any || G.live;
-                }
-                if (!any) break;
-            }
+        if (r >= 3 && r % 2 == 1) {
+            bool any = false;
             for (int k = 0; k < n_groups; ++k) {
                 PassGroup &G = groups[k];
                 if (!G.live) continue;
-                XT_TRY(hipMemcpyAsync(d->host_snap + slot * XT_MAX_LANES + k, &G.lane.cnt->n[qi], sizeof(uint32_t),
-                                      hipMemcpyDeviceToHost, stream_of(k)));
-                XT_TRY(hipEventRecord(d->snap_ev[slot][k], stream_of(k)));
+                uint32_t n = 0;
+                if (r + 1 < G.rounds) {
+                    const int rc = posted(k, n);
+                    if (rc) return rc;
+                }
+                G.live = n != 0;
+                any = any || G.live;
             }
-            slot ^= 1;
-            pending = true;
+            if (!any) break;
         }
     }
     for (int k = 0; after && k < n_groups; ++k) {
@@ -320,27 +329,22 @@ static int render_core(xt_dev *d, const xt_job *job, float *d_out, xt_job_stats 
     if (rc) return rc;
     rc = xt_dev_ensure_accum(d, (size_t)j.W * j.H);
     if (rc) return rc;
-    rc = xt_ensure_host_counters(d);
+    rc = xt_ensure_reports(d);
     if (rc) return rc;
     WaveBuffers &w = d->wave;
     AccumBuffers &a = d->accum;
-    const size_t npix = (size_t)j.W * j.H;
-    const unsigned gfill = grid_for(npix * 4, 256, 8192);
-    hipLaunchKernelGGL(k_fill_u32, dim3(gfill), dim3(256), 0, d->stream, (uint32_t *)a.accf, 0u, npix * 4);
-    hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(npix * 12, 256, 8192)), dim3(256), 0, d->stream,
-                       (uint32_t *)a.acc64, 0u, npix * 12);
+
     // the pixel slots of each group: the slots cut at 8x8 tiles into
     // frame_lanes nearly equal parts (every sample of a pixel stays in its
     // group); one group when a pass hook reads the paths, which it does in
     // the one-group order (path = sample * NT + slot)
     const uint32_t tiles = j.NT / 64;
-    const int n_groups = after_pass ? 1 : (int)std::max(1u, std::min(d->tuning.frame_lanes, tiles));
+    uint32_t want = d->tuning.frame_lanes;
+    if (want == 2 && cap < XT_TWO_GROUPS) want = 1;
+    const int n_groups = after_pass ? 1 : (int)std::max(1u, std::min(want, tiles));
     uint32_t q_at[XT_LANE_STREAMS + 1];
     for (int g = 0; g <= n_groups; ++g) q_at[g] = (uint32_t)((uint64_t)tiles * g / n_groups) * 64u;
-    hipLaunchKernelGGL(k_reset_lanes, dim3(n_groups), dim3(64), 0, d->stream, w.cnt, 0x800000ffu);
-    XT_LAUNCHED();
     d->trace_launches = 0;
-    d->timed_pairs.clear();
     const bool time_trace = stats != nullptr;
     XT_TRY(hipEventRecord(d->ev0, d->stream));
     PassGroup G[XT_LANE_STREAMS];
@@ -354,25 +358,25 @@ static int render_core(xt_dev *d, const xt_job *job, float *d_out, xt_job_stats 
     uint32_t passes = 0;
     for (uint32_t base = 0; base < j.total; base += spp_pass) {
         ++passes;
-        hipLaunchKernelGGL(k_reset_lanes, dim3(n_groups), dim3(64), 0, d->stream, w.cnt, 0x7u);
         // each group's camera rays and accumulation run on the group's own
         // stream, so that they overlap the other groups' rounds (the groups
         // write disjoint pixels)
         const GroupHook camera = [&](int g, hipStream_t st) -> int {
             const WaveLane &L = G[g].lane;
-            hipLaunchKernelGGL(k_set_count, dim3(1), dim3(1), 0, st, L.cnt, 0u, (uint32_t)L.cap);
             Queue q0{w.q[0].r0 + L.off, w.q[0].r1 + L.off, w.q[0].path + L.off};
             hipLaunchKernelGGL(k_camera, dim3(grid_for(L.cap, XT_BLOCK, 8192)), dim3(XT_BLOCK), 0, st, j, base,
                                spp_pass, q_at[g], q_at[g + 1] - q_at[g], (uint32_t)L.off, q0, w.ps0, w.ps1, w.rad,
-                               need64 ? w.ray64 : nullptr, d->tuning.ray_order);
+                               need64 ? w.ray64 : nullptr, d->tuning.ray_order, L.cnt);
             XT_LAUNCHED();
             return XT_OK;
         };
+        const bool last = base + spp_pass >= j.total;
         const GroupHook accumulate = [&](int g, hipStream_t st) -> int {
             const WaveLane &L = G[g].lane;
             hipLaunchKernelGGL(k_accumulate, dim3(grid_for(q_at[g + 1] - q_at[g], XT_BLOCK, 8192)), dim3(XT_BLOCK), 0,
                                st, j, base, spp_pass, q_at[g], q_at[g + 1] - q_at[g], w.rad + L.off,
-                               need64 ? w.ray64 + 6 * L.off : nullptr, a.accf, a.acc64);
+                               need64 ? w.ray64 + 6 * L.off : nullptr, a.accf, a.acc64, base == 0,
+                               last ? (float4 *)d_out : nullptr, L.cnt, last ? d->reports->totals + g : nullptr);
             XT_LAUNCHED();
             return XT_OK;
         };
@@ -383,40 +387,43 @@ static int render_core(xt_dev *d, const xt_job *job, float *d_out, xt_job_stats 
             if (rc) return rc;
         }
     }
-    hipLaunchKernelGGL(k_resolve, dim3(grid_for(npix, XT_BLOCK, 8192)), dim3(XT_BLOCK), 0, d->stream, j, a.accf,
-                       a.acc64, (float4 *)d_out);
-    XT_LAUNCHED();
+    if (j.total == 0) {  // no samples: the image of zero sums
+        hipLaunchKernelGGL(k_accumulate, dim3(grid_for(j.NT, XT_BLOCK, 8192)), dim3(XT_BLOCK), 0, d->stream, j, 0u, 0u,
+                           0u, j.NT, w.rad, (const double *)nullptr, a.accf, a.acc64, true, (float4 *)d_out,
+                           (const Counters *)nullptr, (JobTotals *)nullptr);
+        XT_LAUNCHED();
+    }
     XT_TRY(hipEventRecord(d->ev1, d->stream));
-    XT_TRY(hipMemcpyAsync(d->host_counters, w.cnt, n_groups * sizeof(Counters), hipMemcpyDeviceToHost, d->stream));
     XT_TRY(hipStreamSynchronize(d->stream));
-    for (int g = 1; g < n_groups; ++g) {
-        d->host_counters->queries += d->host_counters[g].queries;
-        d->host_counters->retests += d->host_counters[g].retests;
-        d->host_counters->trace_fail += d->host_counters[g].trace_fail;
-        d->host_counters->steps_exceeded += d->host_counters[g].steps_exceeded;
+    JobTotals sum{};
+    for (int g = 0; g < n_groups && j.total > 0; ++g) {
+        const JobTotals &t = d->reports->totals[g];
+        sum.queries += t.queries;
+        sum.retests += t.retests;
+        sum.trace_fail += t.trace_fail;
+        sum.steps_exceeded += t.steps_exceeded;
     }
     if (stats) {
         std::memset(stats, 0, sizeof *stats);
         float ms = 0.f;
         (void)hipEventElapsedTime(&ms, d->ev0, d->ev1);
         stats->ms_total = ms;
-        stats->queries = d->host_counters->queries;
-        stats->retests = d->host_counters->retests;
-        stats->trace_fail = d->host_counters->trace_fail;
-        stats->retest_fail = d->host_counters->steps_exceeded;
+        stats->queries = sum.queries;
+        stats->retests = sum.retests;
+        stats->trace_fail = sum.trace_fail;
+        stats->retest_fail = sum.steps_exceeded;
         stats->samples = (uint64_t)j.total * j.W * j.H;
         stats->passes = passes;
         // each launch's own time, and the union of the launches' intervals
         // (launches of different groups run at the same time)
         double tsum = 0;
-        std::vector<std::pair<float, float>> spans;
-        for (int k : d->timed_pairs) {
-            float t = 0.f, t0 = 0.f, t1 = 0.f;
-            (void)hipEventElapsedTime(&t, d->tev[k], d->tev[k + 1]);
-            (void)hipEventElapsedTime(&t0, d->ev0, d->tev[k]);
-            (void)hipEventElapsedTime(&t1, d->ev0, d->tev[k + 1]);
-            tsum += t;
-            spans.emplace_back(t0, t1);
+        std::vector<std::pair<double, double>> spans;
+        const uint64_t *at0 = d->reports->stamp;
+        uint64_t zero = ~0ull;
+        for (int k = 0; k < d->trace_launches; ++k) zero = std::min(zero, at0[2 * k]);
+        for (int k = 0; k < d->trace_launches; ++k) {
+            tsum += xt_stamp_ms(d, at0[2 * k], at0[2 * k + 1]);
+            spans.emplace_back(xt_stamp_ms(d, zero, at0[2 * k]), xt_stamp_ms(d, zero, at0[2 * k + 1]));
         }
         std::sort(spans.begin(), spans.end());
         double busy = 0, at = -1e30;
@@ -427,7 +434,7 @@ static int render_core(xt_dev *d, const xt_job *job, float *d_out, xt_job_stats 
         }
         stats->ms_trace = tsum;
         stats->ms_trace_busy = busy;
-        stats->trace_launches = (uint32_t)d->timed_pairs.size();
+        stats->trace_launches = (uint32_t)d->trace_launches;
     }
     return XT_OK;
 }

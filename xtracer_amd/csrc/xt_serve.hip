@@ -478,12 +478,10 @@ int run_pass(xt_dev *d, ServeState &S, const std::vector<Segment> &segs, std::ve
     WaveBuffers &w = d->wave;
     for (size_t g = 0; g < grps.size(); ++g) groups[g].lane.cnt = w.cnt + g;
     XT_TRY(hipEventRecord(S.p0, d->stream));
-    hipLaunchKernelGGL(k_reset_lanes, dim3((unsigned)grps.size()), dim3(64), 0, d->stream, w.cnt, 0x800000ffu);
-    XT_LAUNCHED();
     for (size_t g = 0; g < grps.size(); ++g) {
         const WaveLane &L = groups[g].lane;
         // camera rays fill the lane's queue 0 in slot order
-        hipLaunchKernelGGL(k_set_count, dim3(1), dim3(1), 0, d->stream, L.cnt, 0u, (uint32_t)L.cap);
+        hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, d->stream, L.cnt, (uint32_t)L.cap);
         for (size_t k : grps[g].segs) {
             const SJob &J = S.jobs[segs[k].ticket];
             const size_t n = (size_t)segs[k].samples * segs[k].qn;
@@ -491,7 +489,7 @@ int run_pass(xt_dev *d, ServeState &S, const std::vector<Segment> &segs, std::ve
             Queue q0{w.q[0].r0 + at, w.q[0].r1 + at, w.q[0].path + at};
             hipLaunchKernelGGL(k_camera, dim3(grid_for(n, XT_BLOCK, 8192)), dim3(XT_BLOCK), 0, d->stream, J.jd,
                                J.issued, segs[k].samples, segs[k].q0, segs[k].qn, (uint32_t)at, q0, w.ps0, w.ps1,
-                               w.rad, need64 ? w.ray64 : nullptr, d->tuning.ray_order);
+                               w.rad, need64 ? w.ray64 : nullptr, d->tuning.ray_order, (Counters *)nullptr);
             XT_LAUNCHED();
         }
     }
@@ -501,7 +499,8 @@ int run_pass(xt_dev *d, ServeState &S, const std::vector<Segment> &segs, std::ve
         SJob &J = S.jobs[segs[k].ticket];
         hipLaunchKernelGGL(k_accumulate, dim3(grid_for(segs[k].qn, XT_BLOCK, 8192)), dim3(XT_BLOCK), 0, d->stream,
                            J.jd, J.issued, segs[k].samples, segs[k].q0, segs[k].qn, w.rad + placed[k].path_base,
-                           need64 ? w.ray64 + 6 * placed[k].path_base : nullptr, J.accf, J.acc64);
+                           need64 ? w.ray64 + 6 * placed[k].path_base : nullptr, J.accf, J.acc64, false,
+                           (float4 *)nullptr, (const Counters *)nullptr, (JobTotals *)nullptr);
         XT_LAUNCHED();
         if (segs[k].qn == J.jd.NT) {
             J.issued += segs[k].samples;
@@ -630,7 +629,7 @@ int regen_init(xt_dev *d, ServeState &S) {
     hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(2ull * XT_REGEN_MAX_JOBS * XT_REGEN_SHARDS, 256, 512)), dim3(256), 0,
                        d->stream, (uint32_t *)V.done_shard, 0u, 2ull * XT_REGEN_MAX_JOBS * XT_REGEN_SHARDS);
     hipLaunchKernelGGL(k_regen_init, dim3(1), dim3(1), 0, d->stream, V.ctl, P);
-    hipLaunchKernelGGL(k_reset_lanes, dim3(XT_REGEN_MAX_LANES), dim3(64), 0, d->stream, V.cnt, 0x800000ffu);
+    hipLaunchKernelGGL(k_reset, dim3(XT_REGEN_MAX_LANES), dim3(64), 0, d->stream, V.cnt, 0u);
     XT_LAUNCHED();
     XT_TRY(hipMemcpyAsync(R.lq, R.lq_host, sizeof R.lq_host, hipMemcpyHostToDevice, d->stream));
     XT_TRY(hipMemcpyAsync(R.ls, R.ls_host, sizeof R.ls_host, hipMemcpyHostToDevice, d->stream));
@@ -751,7 +750,7 @@ int regen_lane(xt_dev *d, ServeState &S, const SJob &J, int &lane) {
     L.scene = J.job.scene_id;
     L.integrator = J.jd.integrator;
     L.accel = J.job.accel;
-    hipLaunchKernelGGL(k_reset_lanes, dim3(1), dim3(64), 0, d->stream, R.V.cnt + idle, 0x800000ffu);
+    hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, d->stream, R.V.cnt + idle, 0u);
     XT_LAUNCHED();
     XT_TRY(hipMemcpyAsync(R.lq, R.lq_host, sizeof R.lq_host, hipMemcpyHostToDevice, d->stream));
     XT_TRY(hipMemcpyAsync(R.ls, R.ls_host, sizeof R.ls_host, hipMemcpyHostToDevice, d->stream));
@@ -793,8 +792,6 @@ int regen_round(xt_dev *d, ServeState &S, uint32_t qi) {
         const hipStream_t ls = par ? d->lane_stream[u % ns] : st;
         const DevScene &ds = d->scenes.at(L.scene);
         Counters *cnt = V.cnt + l;
-        hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, ls, cnt,
-                           (1u << (qi ^ 1)) | (1u << CNT_RETEST) | (1u << CNT_CURSOR) | (1u << CNT_RECHECK));
         const Queue in = R.lq_host[qi * XT_REGEN_MAX_LANES + l], out = R.lq_host[(qi ^ 1) * XT_REGEN_MAX_LANES + l];
         TraceBufs B;
         B.q = in;
@@ -804,6 +801,7 @@ int regen_round(xt_dev *d, ServeState &S, uint32_t qi) {
         B.recheck = L.recheck;
         B.cnt = cnt;
         B.cap = R.P;
+        B.par = qi;
         int rc = xt_launch_trace_bufs(d, ds, (int)L.accel, B, nullptr, nullptr, false, ls);
         if (rc) return rc;
         const unsigned g = grid_for(R.P, XT_BLOCK, 8192);

@@ -114,3 +114,26 @@ def test_queue_lengths(device, n):
     device.release(sid)
     assert np.array_equal(got[0].view(np.uint32), ref[0][k].view(np.uint32))
     assert np.array_equal(got[1], ref[1][k])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 3, 64, 1000, 4100, 70000])
+def test_lanes_of_a_ray_agree(device, tmp_path, n):
+    """Short queues leave lanes to walk parts of other lanes' rays: the hits of
+    overlapping, repeated and edge-sharing triangles are those of a queue that
+    keeps every lane busy."""
+    rng = np.random.default_rng(17)
+    c = rng.uniform(-1, 1, (120, 1, 3))
+    tris = c + rng.normal(scale=0.9, size=(120, 3, 3))
+    fan = np.stack([tris[:, 0], tris[:, 2], tris[:, 2] + (tris[:, 1] - tris[:, 0])], axis=1)  # shares edge 0-2
+    s = _soup_scene(tmp_path, np.concatenate([tris, tris, fan, tris[:40]]), [((0.0, 0.0, 0.0), 1.5)])
+    edge = 0.5 * (tris[:, 0] + tris[:, 2])
+    o, d = _rays(1000, 23, np.float32(np.concatenate([tris.mean(axis=1), edge])))
+    sid = device.upload(s)
+    k = np.arange(600000) % len(o)
+    ref = [a[:1000] for a in device.trace(sid, o[k], d[k])[:2]]
+    k = np.arange(n) % len(o)
+    got = device.trace(sid, o[k], d[k])
+    device.release(sid)
+    assert np.array_equal(got[1], ref[1][k])
+    assert np.array_equal(got[0].view(np.uint32), ref[0][k].view(np.uint32))

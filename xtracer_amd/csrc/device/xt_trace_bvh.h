@@ -5,6 +5,15 @@
 // (random rays 2.8 and 0.6, against 11 and 1.2), and the arrays it reads are
 // 63 MB of triangles and 18 MB of nodes, against 289 MB and 54 MB.
 //
+// Once the queue is empty, idle lanes help: one takes the siblings that a
+// walking lane has not visited yet, or the top of its stack, walks them with the
+// ray's state and hands its closest hit back; the lanes of a ray share the
+// closest distance. What bounds a queue of fewer rays than the card has lanes is
+// the chain of dependent loads of the rays with the longest walks, and this
+// shares them out: 100,003 terrain camera rays 115 to 86 us, a 333x211 depth
+// frame 236 to 191, 256x256x4 paths 715 to 560, and the end of larger launches
+// (4 M random rays 710 to 545, 1080p 16 spp paths 16.2 to 15.0 ms).
+//
 // Bound by VALU issue (80% of the time on the 1080p icosphere frame). What it
 // measured, trace time of that frame's 72.1 M queries with the launches one
 // after another: kd-tree walk 15.5 ms, this 9.4 ms; 4 M random rays 1256 to
@@ -14,6 +23,7 @@
 #include "xt_walk.h"
 
 #define XT_W_KEEP 6    // sixteenths of the working lanes at which a phase of a turn ends (3: 3% slower, 8: 1%)
+#define XT_W_FREE 32   // walked rays of a wave at which they are finished for their lanes to help (8: 4% slower at 72 K rays)
 #define XT_W_WAVES 4   // waves per SIMD: as many as the LDS of 10 KB a wave leaves room for
 
 // Gathers records of PARTS 16-byte parts into LDS: record `rec` (an index) of
@@ -56,6 +66,31 @@ __device__ __forceinline__ void gather_records(const void *base, uint32_t rec, u
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
+// A helper's result into its ray's: the closest hit as one more candidate, and
+// what the helper deferred. The ray's decisions stay what they would be for one
+// lane: candidates within the tie band go to the FP64 re-check.
+__device__ __forceinline__ void merge_best(Best &b, uint32_t &rec, float t, uint32_t prim, uint32_t prec, float mark_t,
+                                           uint32_t c0, uint32_t c1) {
+    if (prim != XT_NONE) {
+        const uint32_t was = b.prim;
+        offer(b, t, prim);
+        rec = b.prim != was ? prec : rec;
+    }
+    if (c0 != XT_NONE) defer(b, mark_t, c0);
+    if (c1 == XT_CAND_OVERFLOW) b.c1 = c1;
+    else if (c1 != XT_NONE) defer(b, mark_t, c1);
+}
+
+__device__ __forceinline__ float from_lane(float v, uint32_t src) {
+    return __int_as_float(__builtin_amdgcn_ds_bpermute((int)(src << 2), __float_as_int(v)));
+}
+__device__ __forceinline__ uint32_t from_lane(uint32_t v, uint32_t src) {
+    return (uint32_t)__builtin_amdgcn_ds_bpermute((int)(src << 2), (int)v);
+}
+__device__ __forceinline__ float lane_value(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 
 // STACK: the deepest a walk's stack gets, which the tree's depth bounds. A
@@ -93,23 +128,58 @@ static __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(XT_W_
     uint32_t tbase = 0, lhit = 0, lmask = 0;  // leaf children hit and not yet tested, the node's leaves
     uint32_t tk = 0, tn = 0, best_rec = 0;    // primitives of the leaf in hand; the closest one's record
     uint32_t sp = 0;
+    uint32_t own = lane;        // the lane whose ray this one walks
+    float shared_t = INFINITY;  // closest hit of the ray's other lanes, when last seen
 
     for (;;) {
         int nw = __popcll(__builtin_amdgcn_ballot_w64(alive));
-        if (nw == 0 || (more && 64 - nw >= XT_REFILL_IDLE)) {
-            if (__builtin_amdgcn_ballot_w64(done)) {
-                bool mark = false, full = false;
-                if (done)
-                    finish_ray(S, in, hit, cnt, ri, o, origin, true, best, recs, best_rec, mark, full);
-                if (__builtin_amdgcn_ballot_w64(mark)) {
-                    const bool rf = mark && full, rc = mark && !full;
-                    const uint32_t slot = wave_append(rf, &cnt->n[CNT_RETEST + T.par]);
-                    if (rf) retest_list[slot] = ri;
-                    const uint32_t cslot = wave_append(rc, &cnt->n[CNT_RECHECK + T.par]);
-                    if (rc) recheck_list[cslot] = make_uint4(ri, best.c0, best.c1, XT_NONE);
+        const bool low = nw == 0 || (more && 64 - nw >= XT_REFILL_IDLE);
+        bool fin = done && low;
+        if (!more) {
+            // what helpers without work have found goes to their rays
+            unsigned long long hm = __builtin_amdgcn_ballot_w64(done && own != lane);
+            if (hm) {
+                do {
+                    const int h = __builtin_ctzll(hm);
+                    hm &= hm - 1ull;
+                    const uint32_t to = __builtin_amdgcn_readlane(own, h);
+                    const float t = lane_value(best.t, h), mt = lane_value(best.mark_t, h);
+                    const uint32_t prim = __builtin_amdgcn_readlane(best.prim, h);
+                    const uint32_t rec = __builtin_amdgcn_readlane(best_rec, h);
+                    const uint32_t c0 = __builtin_amdgcn_readlane(best.c0, h);
+                    const uint32_t c1 = __builtin_amdgcn_readlane(best.c1, h);
+                    if (lane == to) merge_best(best, best_rec, t, prim, rec, mt, c0, c1);
+                } while (hm);
+                if (own != lane) {
+                    done = false;
+                    own = alive ? own : lane;
                 }
-                done = false;
             }
+            fin = done && nw == 0;
+            // rays that no helper walks any more are finished, for their lanes to help
+            if (nw != 0 && __popcll(__builtin_amdgcn_ballot_w64(done)) >= XT_W_FREE) {
+                unsigned long long busy = __builtin_amdgcn_ballot_w64(alive && own != lane), kept = 0;
+                while (busy) {
+                    kept |= 1ull << __builtin_amdgcn_readlane(own, __builtin_ctzll(busy));
+                    busy &= busy - 1ull;
+                }
+                fin = done && !((kept >> lane) & 1ull);
+            }
+        }
+        if (__builtin_amdgcn_ballot_w64(fin)) {
+            bool mark = false, full = false;
+            if (fin)
+                finish_ray(S, in, hit, cnt, ri, o, origin, true, best, recs, best_rec, mark, full);
+            if (__builtin_amdgcn_ballot_w64(mark)) {
+                const bool rf = mark && full, rc = mark && !full;
+                const uint32_t slot = wave_append(rf, &cnt->n[CNT_RETEST + T.par]);
+                if (rf) retest_list[slot] = ri;
+                const uint32_t cslot = wave_append(rc, &cnt->n[CNT_RECHECK + T.par]);
+                if (rc) recheck_list[cslot] = make_uint4(ri, best.c0, best.c1, XT_NONE);
+            }
+            done = done && !fin;
+        }
+        if (low) {
             while (more) {
                 const bool idle = !alive && !done;
                 const unsigned long long m = __builtin_amdgcn_ballot_w64(idle);
@@ -149,6 +219,7 @@ static __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(XT_W_
                         grp = 1u << oct;
                         lhit = tn = 0;
                         sp = 0;
+                        shared_t = INFINITY;
                         // a ray of no direction meets no triangle and no sphere
                         alive = dk != 0.f;
                         done = !alive;
@@ -157,10 +228,74 @@ static __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(XT_W_
                 R.cur += left < free_lanes ? left : free_lanes;
             }
             nw = __popcll(__builtin_amdgcn_ballot_w64(alive));
-            if (nw == 0) {
-                if (!more && !__builtin_amdgcn_ballot_w64(done)) break;
-                continue;
+        }
+        if (!more && nw != 0) {
+            // no ray is left: idle lanes take over parts of the walking lanes' trees
+            const bool idle = !alive && !done;
+            const uint32_t bits = (uint32_t)__popc(grp & 0xffu);
+            const bool can = alive && (bits >= 2u || sp != 0u || ((lhit | tn) != 0u && grp != 0u));
+            const unsigned long long im = __builtin_amdgcn_ballot_w64(idle), dm = __builtin_amdgcn_ballot_w64(can);
+            if (im && dm) {
+                const uint32_t ni = (uint32_t)__popcll(im), nd = (uint32_t)__popcll(dm), pairs = ni < nd ? ni : nd;
+                const uint32_t ri_ = rank_in(im), rd = rank_in(dm);
+                const bool give = can && rd < pairs, take = idle && ri_ < pairs;
+                uint32_t gift = 0;
+                if (give) {
+                    if (bits >= 2u) {  // the siblings after the next one
+                        const uint32_t low = grp & (0u - grp);
+                        gift = grp ^ low;
+                        grp = (grp & ~0xffu) | low;
+                    } else if (sp) {
+                        sp -= BS;
+                        gift = stk[sp];
+                    } else {
+                        gift = grp;
+                        grp = 0;
+                    }
+                }
+                // lane r of `giver` holds the lane of rank r among the givers (at most 32)
+                const uint32_t giver = (uint32_t)__builtin_amdgcn_ds_permute((int)((give ? rd : 63u) << 2), (int)lane);
+                const uint32_t from = from_lane(giver, take ? ri_ : 63u);
+                const uint32_t src = take ? from : lane;
+                gift = from_lane(gift, src);
+                const uint32_t pk = from_lane(oct | kz << 3 | own << 5, src);
+                ri = from_lane(ri, src);
+                origin = from_lane(origin, src);
+                o = mk(from_lane(o.x, src), from_lane(o.y, src), from_lane(o.z, src));
+                inv = mk(from_lane(inv.x, src), from_lane(inv.y, src), from_lane(inv.z, src));
+                eta = mk(from_lane(eta.x, src), from_lane(eta.y, src), from_lane(eta.z, src));
+                sx = from_lane(sx, src);
+                sy = from_lane(sy, src);
+                sz = from_lane(sz, src);
+                best.t = from_lane(best.t, src);
+                best.prim = from_lane(best.prim, src);
+                best_rec = from_lane(best_rec, src);
+                if (take) {
+                    oct = pk & 7u;
+                    kz = (pk >> 3) & 3u;
+                    own = pk >> 5;
+                    best.mark_t = INFINITY;
+                    best.c0 = best.c1 = XT_NONE;
+                    grp = gift;
+                    lhit = tn = sp = 0;
+                    alive = true;
+                }
             }
+            if (__builtin_amdgcn_ballot_w64(alive && own != lane)) {
+                // the closest hit of all lanes of a ray ends each one's walk
+                int *const tm = (int *)buf;
+                tm[lane] = __float_as_int(INFINITY);
+                __builtin_amdgcn_wave_barrier();
+                if (alive || done) atomicMin(tm + own, __float_as_int(best.t));
+                __builtin_amdgcn_wave_barrier();
+                shared_t = __int_as_float(tm[own]);
+                asm volatile("" ::"v"(shared_t) : "memory");
+            }
+            nw = __popcll(__builtin_amdgcn_ballot_w64(alive));
+        }
+        if (nw == 0) {
+            if (!more && !__builtin_amdgcn_ballot_w64(done)) break;
+            continue;
         }
         const int keep = (nw * XT_W_KEEP) >> 4;
 
@@ -191,7 +326,7 @@ static __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(XT_W_
                 const float anx = px * inv.x - eta.x, afx = px * inv.x + eta.x;
                 const float any_ = py * inv.y - eta.y, afy = py * inv.y + eta.y;
                 const float anz = pz * inv.z - eta.z, afz = pz * inv.z + eta.z;
-                const float lim = best.t * (1.f + 4e-6f);
+                const float lim = fminf(best.t, shared_t) * (1.f + 4e-6f);
                 uint32_t hits = 0;
 #pragma unroll
                 for (int c = 0; c < 8; ++c) {
@@ -259,7 +394,7 @@ static __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(XT_W_
                 if (prim != origin) {
                     const uint32_t was = best.prim;
                     if (XT_PRIM_TYPE(__float_as_uint(a.w)) == XT_PRIM_TRIANGLE) {
-                        tri32_flat(o, sx, sy, sz, kz, a, b, c, prim, best);
+                        tri32_flat<true>(o, sx, sy, sz, kz, a, b, c, prim, best, inv, eta);
                     } else {
                         const float4 b4 = in.r1[ri];
                         sph32(o, mk(b4.x, b4.y, b4.z), tsmall_of(o), a, b, prim, best);

@@ -167,7 +167,7 @@ static __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(XT_KD
                 leaf = payload != 0u;
                 if (prim != origin) {
                     if (XT_PRIM_TYPE(__float_as_uint(a.w)) == XT_PRIM_TRIANGLE) {
-                        tri32_flat(o, sx, sy, sz, kz, a, b, c, prim, best);
+                        tri32_flat<false>(o, sx, sy, sz, kz, a, b, c, prim, best, inv, inv);
                     } else {
                         const float4 b4 = in.r1[ri];
                         sph32(o, mk(b4.x, b4.y, b4.z), tsmall_of(o), a, b, prim, best);

@@ -7,8 +7,11 @@
 #define XT_RUN_MAX 512u     // rays of the longest run a wave takes at once
 #define XT_REFILL_IDLE 24   // a wave takes new rays once this many lanes are idle
 
-// Where a wave's rays come from. Wave w first takes rays [64 w, 64 w + 64);
-// the rays beyond 64 times the grid's waves are cut into stretches of 2^sh
+// Where a wave's rays come from. Wave w first takes 64 consecutive rays, or, when
+// the grid's waves could take more than there are, its equal share of them: the
+// rays of a wave wait for each other's phases, and its idle lanes help (256x256x4
+// paths 715 us with 64 a wave, 660 with equal shares). The rays beyond 64 times
+// the grid's waves are cut into stretches of 2^sh
 // dealt to the XCDs in turn (nseg = 8: one stretch each), each XCD's stretches
 // with a cursor in a line of its own. A wave takes runs from its own XCD's
 // cursor, shorter ones as the end comes near, and then from the others'.
@@ -20,7 +23,7 @@
 // runs of up to 512 rays leave 0.1 ms; a queue that one run per wave covers
 // needs no atomic at all (100,003 rays: 219 to 120 us).
 struct RaySource {
-    uint32_t n, base, sh, len, par, xcd;  // rays, first dealt ray, log2 of a stretch (or, sh = 32, its length)
+    uint32_t n, first, base, sh, len, par, xcd;  // rays, first dealt ray, log2 of a stretch (or, sh = 32, its length)
     uint32_t waves;                  // per XCD
     uint32_t cur, end;               // the run in hand: rays (first run), or positions on the XCD's stretches
     uint32_t seen;                   // the XCD's cursor when last seen
@@ -31,7 +34,8 @@ __device__ __forceinline__ void source_init(RaySource &R, uint32_t n, uint32_t w
     const uint32_t nseg = T.nseg;
     R.n = n;
     R.par = T.par;
-    R.base = waves * 64u < n ? waves * 64u : n;
+    R.first = waves * 64u < n ? 64u : (n + waves - 1u) / waves;
+    R.base = waves * R.first < n ? waves * R.first : n;
     R.sh = nseg == 1u ? (uint32_t)XT_STRETCH_LOG : 32u;
     R.len = nseg == 1u ? 1u << XT_STRETCH_LOG : ((n - R.base) / 8u + 64u) & ~63u;
     R.xcd = __builtin_amdgcn_s_getreg(20 | 3 << 11) & 7u;  // XCC_ID
@@ -58,8 +62,8 @@ __device__ __forceinline__ uint32_t source_ray(const RaySource &R, uint32_t at) 
 __device__ __forceinline__ bool source_next(RaySource &R, Counters *cnt, uint32_t wave) {
     if (R.state == 0u) {
         R.state = 1u;
-        R.cur = wave * 64u < R.n ? wave * 64u : R.n;
-        R.end = R.n - R.cur < 64u ? R.n : R.cur + 64u;
+        R.cur = wave * R.first < R.n ? wave * R.first : R.n;
+        R.end = R.n - R.cur < R.first ? R.n : R.cur + R.first;
         if (R.cur < R.end) return true;
     }
     R.state = 2u;
@@ -143,10 +147,31 @@ __device__ __forceinline__ float ray_shear(f3 d, uint32_t &kz, float &sx, float 
     return dk;
 }
 
+// Where the ray enters the triangle's box, widened by half of eta; INFINITY
+// when it passes it by.
+__device__ __forceinline__ float tri_box_entry(f3 A, f3 B, f3 C, f3 inv, f3 eta) {
+    float t0 = 0.f, t1 = INFINITY;
+    const float v[3][3] = {{A.x, B.x, C.x}, {A.y, B.y, C.y}, {A.z, B.z, C.z}};
+    const float iv[3] = {inv.x, inv.y, inv.z}, e[3] = {eta.x, eta.y, eta.z};
+    for (int k = 0; k < 3; ++k) {
+        const float p = fminf(v[k][0], fminf(v[k][1], v[k][2])) * iv[k];
+        const float q = fmaxf(v[k][0], fmaxf(v[k][1], v[k][2])) * iv[k];
+        t0 = fmaxf(t0, fminf(p, q) - 0.5f * e[k]);
+        t1 = fminf(t1, fmaxf(p, q) + 0.5f * e[k]);
+    }
+    return t0 <= t1 ? t0 : INFINITY;
+}
+
 // tri32 and offer() in one straight line: the tests' rare outcomes (a
-// deferral) share one branch. Same decisions, in the same order.
+// deferral) share one branch. Same decisions, in the same order; but with BOX a
+// grazed triangle is deferred from where the ray enters its box (rinv, eta: the
+// ray's reciprocal direction and the slack of the walk's boxes) and not from the ray's origin: a walk that visits
+// the tree in another order, and so tests other triangles behind the closest
+// hit, decides alike which rays are re-checked.
+template <bool BOX>
 __device__ __forceinline__ void tri32_flat(const f3 o, float sx, float sy, float sz, uint32_t kz, const float4 a,
-                                           const float4 b, const float4 c, uint32_t prim, Best &best) {
+                                           const float4 b, const float4 c, uint32_t prim, Best &best, f3 rinv,
+                                           f3 eta) {
     const uint32_t tf = __float_as_uint(a.w);
     const float tsmall = tsmall_of(o);
     const f3 A = sub(mk(a.x, a.y, a.z), o), B = sub(mk(b.x, b.y, b.z), o), C = sub(mk(c.x, c.y, c.z), o);
@@ -177,7 +202,8 @@ __device__ __forceinline__ void tri32_flat(const f3 o, float sx, float sy, float
     }
     if (rare) {
         if (graze) {
-            defer(best, 0.f, prim);
+            const float at = BOX ? tri_box_entry(A, B, C, rinv, eta) : 0.f;
+            if (at < INFINITY) defer(best, at, prim);
         } else {
             if (m > -XT_BAND && m < XT_BAND) defer(best, t, prim);
             if (in && near0) defer(best, fmaxf(t, 0.f), prim);

@@ -475,7 +475,7 @@ static void launch_kd_trace_sb(unsigned per_cu, int n_cu, size_t cap, hipStream_
         }
         per_cu = (unsigned)resident;
     }
-    const size_t need = (cap + BS - 1) / BS;
+    const size_t need = (cap + BS / 64 - 1) / (BS / 64);  // a wave for every ray
     const unsigned g = (unsigned)std::max<size_t>(1, std::min<size_t>(need, (size_t)n_cu * per_cu));
     hipLaunchKernelGGL((k_trace_kd<STACK, BS>), dim3(g), dim3(BS), 0, st, v, q, count, hit, retest, recheck, T);
 }
@@ -494,7 +494,7 @@ static void launch_bvh_trace_sb(unsigned per_cu, int n_cu, size_t cap, hipStream
         }
         per_cu = (unsigned)resident;
     }
-    const size_t need = (cap + BS - 1) / BS;
+    const size_t need = (cap + BS / 64 - 1) / (BS / 64);  // a wave for every ray
     const unsigned g = (unsigned)std::max<size_t>(1, std::min<size_t>(need, (size_t)n_cu * per_cu));
     hipLaunchKernelGGL((k_trace_bvh<STACK, BS>), dim3(g), dim3(BS), 0, st, v, q, count, hit, retest, recheck, T);
 }

@@ -176,3 +176,21 @@ def test_rebuild_refused_while_served(device):
     assert done
     device.build_kd(sid)  # idle again: rebuilt
     device.release(sid)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 255, 256, 257, 513, 1500])
+def test_overlapping_soups(device, tmp_path, n):
+    """Large overlapping triangles, most of them cut by every plane: references
+    and clips around the edges of a wave and of its stretch of references."""
+    rng = np.random.default_rng(n)
+    tris = rng.uniform(-1, 1, (n, 1, 3)) + rng.normal(scale=0.6, size=(n, 3, 3))
+    scn.write_obj(tmp_path / "soup.obj", tris)
+    path = scn.write(tmp_path / "scene.scn", {"soup": dict(type="mesh", source="soup.obj"),
+                                              "ball": dict(type="sphere", position=(0.0, 0.0, 0.0), radius=0.75)},
+                     {"soup": ("soup", "m"), "ball": ("ball", "m")}, {"m": dict(type="lambert", kd=(0.5, 0.5, 0.5))})
+    host = xa.Scene(path, threads=1)
+    sid = device.upload(host)
+    device.build_kd(sid)
+    _same_tree(device, sid, host, f"{n} overlapping triangles")
+    device.release(sid)

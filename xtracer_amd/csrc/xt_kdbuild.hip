@@ -230,7 +230,7 @@ int build(xt_dev *d, const SceneView &v, const xt_build_params *bp, XtScratch &m
         hipLaunchKernelGGL(k_kdb_sah, dim3((NL + 3) / 4), dim3(256), 0, d->stream, nd, NL, NR, level, P,
                            (const int32_t *)as<int32_t>(big_of), (const uint32_t *)as<uint32_t>(gbins), a0, a1,
                            as<int2>(split));
-        hipLaunchKernelGGL(k_kdb_classify, dim3(grid_for(NR, 256, 16384)), dim3(256), 0, d->stream, a0, a1, NR, nd, NL,
+        hipLaunchKernelGGL(k_kdb_classify, dim3(grid_for(NR, XT_KDB_CLASSIFY, 16384)), dim3(64), 0, d->stream, a0, a1, NR, nd, NL,
                            (const int2 *)as<int2>(split), v.prims, v.prims64, n, as<uint64_t>(flags), as<float4>(l0),
                            as<float4>(l1), as<float4>(q0), as<float4>(q1), as<KdbCtl>(ctl));
         XT_LAUNCHED();

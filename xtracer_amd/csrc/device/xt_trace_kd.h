@@ -5,12 +5,12 @@
 // their hits are written and they get new rays. With whole groups of 64 rays
 // a wave ran as long as its longest ray: 10 of 64 lanes were active in the mean
 // instruction (1080p icosphere frame, rocprofv3), 26 with the refill. The
-// turn's phases end at a quarter of the working lanes: later (1/8) and earlier
-// (1/2) were 2% and 7% slower on the strands frame.
+// turn's phases end at 3 sixteenths of the working lanes: 4 and 6 were 1.6% and
+// 7% slower on the strands frame (23.2 ms).
 #pragma once
 #include "xt_walk.h"
 
-#define XT_KD_KEEP 4      // sixteenths of the working lanes at which a phase ends
+#define XT_KD_KEEP 3      // sixteenths of the working lanes at which a phase ends
 #define XT_KD_WAVES 5     // waves per SIMD (96 VGPRs; at 6, with 88 B of spills, 3% slower)
 #define XT_KD_EPS 2e-6f   // relative widening of the walk's intervals
 

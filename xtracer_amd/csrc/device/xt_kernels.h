@@ -360,6 +360,13 @@ static __global__ __launch_bounds__(XT_BLOCK) void k_camera(const JobDev j, uint
     if (cnt && blockIdx.x == 0) reset_counters(cnt, n, pass_base == 0);
     const uint32_t stride = gridDim.x * blockDim.x;
     const uint32_t qword = 1u | (j.rdepth << 16);
+    // bound by its stores (84 bytes a path with all state), so only the
+    // state that the integrator's shading reads: the pathtracer all of it, ao
+    // the random key. Every path's shading stores its radiance, unless there is
+    // no round.
+    const bool set_s1 = j.integrator == XT_INTEGRATOR_PATHTRACER;
+    const bool set_s0 = set_s1 || j.integrator == XT_INTEGRATOR_AO;
+    const bool set_rad = set_s1 && j.rdepth == 0;
     // order 2 (with whole tiles): queue entry i holds sample sl of slot w of
     // tile t, i = (t * spp_pass + sl) * 64 + w, so that a stretch of the
     // queue covers one part of the image; order 3: the pass's samples of one
@@ -385,7 +392,7 @@ static __global__ __launch_bounds__(XT_BLOCK) void k_camera(const JobDev j, uint
         const uint32_t s = pass_base + sl;
         uint32_t x = 0, y = 0;
         const bool live = slot_pixel(j, q, x, y) && s < j.total;
-        rad[path] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (set_rad) rad[path] = make_float4(0.f, 0.f, 0.f, 0.f);
         out.path[i] = path;
         if (!live) {
             out.r0[i] = make_float4(0.f, 0.f, 0.f, __uint_as_float(XT_DEAD));
@@ -398,8 +405,8 @@ static __global__ __launch_bounds__(XT_BLOCK) void k_camera(const JobDev j, uint
         float cx, cy;
         aa_coords(j, x, y, s / j.spp, cx, cy);
         camera_ray(j, cx, cy, key, o, d);
-        ps0[path] = make_float4(1.f, 1.f, 1.f, __uint_as_float(key));
-        ps1[path] = make_float4(1.f, 1.f, 1.f, __uint_as_float(qword));
+        if (set_s0) ps0[path] = make_float4(1.f, 1.f, 1.f, __uint_as_float(key));
+        if (set_s1) ps1[path] = make_float4(1.f, 1.f, 1.f, __uint_as_float(qword));
         if (ray64) {
             double *r = ray64 + 6 * (size_t)path;
             r[0] = o[0];

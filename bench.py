@@ -133,7 +133,7 @@ def traffic_probe(args):
                         "stderr_tail": r.stderr[-400:]}
             queries.append(json.loads(lines[-1])["extra"]["queries_per_frame"] * 2)
             for name, ctr, val in _counter_rows(out):
-                if name.split("<")[0].split("(")[0].strip().endswith(TRACE_KERNEL):
+                if TRACE_KERNEL in name.split("<")[0].split("(")[0]:
                     sums[ctr] = sums.get(ctr, 0.0) + val
                 elif COPY_KERNEL in name:
                     copy[ctr] = max(copy.get(ctr, 0.0), val)
@@ -550,7 +550,7 @@ def main():
                      "traffic_per_query": probe.get("bytes_per_query") if probe else None,
                      "l2_hit_rate": probe.get("l2_hit_rate") if probe else None,
                      "traffic_probe": probe,
-                     "kernel": "k_trace (kd-tree)", "bytes_per_query": TRACE_BYTES_PER_QUERY,
+                     "kernel": "k_trace_bvh (wide BVH)", "bytes_per_query": TRACE_BYTES_PER_QUERY,
                      "avg_launch_ms": round(trace_ms / max(1, launches), 4), "launches": launches,
                      "busy_ms_per_frame": round(busy_ms / max(1, args.steps), 3),
                      "concurrent_groups": tuning.get("frame_lanes", 1),

@@ -230,7 +230,8 @@ const char *xt_last_error(const xt_dev *d);
  * force (trace_blocks_per_cu 0: as many blocks as a CU keeps resident). */
 #define XT_TUNING_AUTO 0xffffffffu /* trace_blocks_per_cu: back to resident fill */
 typedef struct xt_tuning {
-    uint32_t kd_stack;        /* kd short-stack entries per lane: 8, 12, 16 or 24 (12) */
+    uint32_t kd_stack;        /* kd short-stack entries per lane: 8, 12, 16 or 24 (12); scenes
+                                 walked on the wide BVH take what its depth needs */
     uint32_t trace_block;     /* lanes per trace block: 128 or 256 (256) */
     uint32_t wave_paths;      /* paths in flight per wavefront pass, 4096..2^28 (64M: a 1080p 16 spp frame in one pass) */
     uint32_t trace_blocks_per_cu; /* persistent trace grid: blocks per CU, <= 64 (resident fill) */
@@ -240,12 +241,13 @@ typedef struct xt_tuning {
                                  an 8x8 tile together; 3 all samples of a pixel together (1) */
     uint32_t kd_layout;       /* kd-tree node order of scenes uploaded afterwards: 1 depth-first; 2 child
                                  pairs grouped into 128-byte lines three levels deep (1) */
-    uint32_t kd_leaf;         /* kd leaf primitives in the FP32 walk: 1 a copy of each referenced record in
+    uint32_t kd_leaf;         /* leaf primitives in the FP32 walk: 1 a copy of each referenced record in
                                  leaf order; 2 read from the soup through the reference list (1) */
     uint32_t frame_lanes;     /* one-job renders: 1 a pass's paths in one group on the device stream; 2..4
                                  its pixels cut into that many groups whose rounds run on streams of their
                                  own, so that one group's shading and launch tails overlap another's trace;
-                                 images are the same bits either way (2) */
+                                 images are the same bits either way; 2 leaves passes below 2^19 paths
+                                 in one group (2) */
 } xt_tuning;
 int xt_dev_set_tuning(xt_dev *d, const xt_tuning *t);
 int xt_dev_get_tuning(const xt_dev *d, xt_tuning *t);

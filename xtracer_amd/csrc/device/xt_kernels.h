@@ -1,11 +1,12 @@
 // Wavefront kernels. One "pass" renders `spp_pass` samples of every pixel:
-//   k_camera  -> queue of camera rays (compacted), path state, zeroed radiance
+//   k_camera  -> queue of camera rays (compacted), path state, counters
 //   repeat per query index q = 1..rdepth:
-//     k_trace   FP32 closest hit per queued ray, rays needing the FP64 re-test
-//               appended to a list
-//     k_retest  FP64 re-trace of the listed rays with the reference predicates
+//     k_trace_* FP32 closest hit per queued ray (k_trace_bvh, k_trace_kd or
+//               k_trace_oct), rays needing an FP64 decision appended to lists
+//     k_recheck FP64 re-check and re-test of the listed rays with the
+//               reference predicates
 //     k_shade_* integrator rule; surviving paths appended (ballot + prefix
-//               sum, one atomic per wave) to the next queue
+//               sum, one atomic per block) to the next queue
 //   k_accumulate  per-pixel sum over the pass's samples in sample order
 // Every kernel reads its work count from device memory and loops over it, so
 // the launch sequence is fixed and can be captured in a hipGraph.
@@ -950,11 +951,16 @@ static __global__ __launch_bounds__(XT_BLOCK) void k_shade_pt(const SceneView S,
 }
 
 // AO, first query (src/xtcore/integrator/ao/integrator.cc:12-53): a hit
-// spawns one hemisphere ray; a miss scores w = 1.
-static __global__ __launch_bounds__(XT_BLOCK) void k_shade_ao1(const SceneView S, const Queue in,
+// spawns one hemisphere ray; a miss scores w = 1. Paced by the appends, atomics
+// on one address of about 11 ns each: blocks of 1024 lanes make a quarter of
+// those of 256 (512x512x16 frame 955 to 876 us). The pathtracer's step, which
+// has more to do per ray and shares the card with the other group's trace,
+// stays at 256 (1024: strands frame 23.1 to 23.9 ms).
+#define XT_AO_BLOCK 1024
+static __global__ __launch_bounds__(XT_AO_BLOCK) void k_shade_ao1(const SceneView S, const Queue in,
                                                         const uint32_t *in_count, const float4 *hit, Queue out,
                                                         uint32_t *out_count, const float4 *ps0, float4 *rad) {
-    __shared__ uint32_t lds[XT_BLOCK / 64 + 1];
+    __shared__ uint32_t lds[XT_AO_BLOCK / 64 + 1];
     const uint32_t n = *in_count;
     const uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += stride) {
@@ -984,7 +990,7 @@ static __global__ __launch_bounds__(XT_BLOCK) void k_shade_ao1(const SceneView S
                 nself = self_hit_t(g, N, dir);
             }
         }
-        const uint32_t slot = block_append<XT_BLOCK>(cont, out_count, lds);
+        const uint32_t slot = block_append<XT_AO_BLOCK>(cont, out_count, lds);
         if (cont) push_ray(out, slot, no, nd, nprim, nself, path);
     }
 }

@@ -167,8 +167,8 @@ int xt_launch_shade(xt_dev *d, const DevScene &ds, uint32_t integrator, uint32_t
             break;
         case XT_INTEGRATOR_AO:
             if (r == 0)
-                hipLaunchKernelGGL(k_shade_ao1, dim3(g), dim3(XT_BLOCK), 0, st, ds.view, in, n_in, hit, out,
-                                   n_out, w.ps0, w.rad);
+                hipLaunchKernelGGL(k_shade_ao1, dim3(grid_for(L.cap, XT_AO_BLOCK, 2048)), dim3(XT_AO_BLOCK), 0, st,
+                                   ds.view, in, n_in, hit, out, n_out, w.ps0, w.rad);
             else
                 hipLaunchKernelGGL(k_shade_ao2, dim3(g), dim3(XT_BLOCK), 0, st, in, n_in, hit, w.rad);
             break;

@@ -10,7 +10,7 @@
 //                  queue)
 //   k_regen_gen    camera rays of the new segments, appended to each lane's
 //                  queue behind the paths that are still running
-//   per lane       k_trace / k_recheck / k_retest as for one job, then the
+//   per lane       the trace and k_recheck as for one job, then the
 //                  shading step; a path that continues is appended to the
 //                  lane's next queue, one that ends to the retire list
 //   k_regen_retire each ended path's radiance stored in its job's sample

@@ -28,7 +28,6 @@ static __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(XT_KD
     uint2 *const stk = kstk + threadIdx.x;
     const uint32_t n = *in_count;
     trace_open(T, n);
-    const uint32_t lane = lane_id();
     const uint32_t waves = gridDim.x * (BS / 64);
     const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (BS / 64) + (threadIdx.x >> 6));
     RaySource R;

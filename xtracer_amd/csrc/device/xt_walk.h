@@ -107,7 +107,7 @@ __device__ __forceinline__ uint32_t rank_in(unsigned long long m) {
 
 // Writes a walked ray's hit: the closest triangle's t and barycentrics in
 // FP64, or the FP32 record of a ray whose deferred candidates the FP64
-// kernels decide; `mark` and `full` as k_recheck and k_retest take them.
+// kernel decides: `mark` lists it, `full` for the whole re-test.
 // recs[3 rec ..] is the closest primitive's record, if it is a primitive.
 __device__ __forceinline__ void finish_ray(const SceneView &S, const Queue &in, float4 *hit, Counters *cnt,
                                            uint32_t ri, f3 o, uint32_t origin, bool ok, const Best &best,

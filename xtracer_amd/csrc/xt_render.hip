@@ -242,11 +242,14 @@ int xt_run_rounds(xt_dev *d, PassGroup *groups, int n_groups, bool time_trace, c
     struct Join {
         xt_dev *d;
         int n_st;
+        bool failed = true;  // a trace still queued may post a count: none is left to the next call
         ~Join() {
+            if (failed) (void)hipStreamSynchronize(d->stream);
             for (int k = 0; k < n_st; ++k) {
                 if (hipEventRecord(d->lane_ev[k], d->lane_stream[k]) != hipSuccess ||
                     hipStreamWaitEvent(d->stream, d->lane_ev[k], 0) != hipSuccess)
                     (void)hipStreamSynchronize(d->lane_stream[k]);
+                if (failed) (void)hipStreamSynchronize(d->lane_stream[k]);
             }
         }
     } join{d, n_st};
@@ -306,6 +309,7 @@ int xt_run_rounds(xt_dev *d, PassGroup *groups, int n_groups, bool time_trace, c
         const int rc = (*after)(k, stream_of(k));
         if (rc) return rc;
     }
+    join.failed = false;
     return XT_OK;
 }
 

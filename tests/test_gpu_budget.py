@@ -1,0 +1,68 @@
+"""Scenes at the limit of a device's HBM budget."""
+import numpy as np
+import pytest
+
+import xtracer_amd as xa
+from tests.helpers import HipBuffers, mixed_rays, scene_path
+
+E_BUDGET = 5
+
+
+class Rays:
+    """Device-resident rays for the trace that allocates nothing."""
+
+    def __init__(self, n, box):
+        o, d = mixed_rays(None, n, seed=11, box=box)
+        r0, r1 = np.zeros((n, 4), np.float32), np.zeros((n, 4), np.float32)
+        r0[:, :3], r1[:, :3] = o, d
+        r0[:, 3] = np.uint32(xa.HIT_NONE).view(np.float32)
+        self.n, self.hip = n, HipBuffers()
+        self.r0, self.r1, self.out = self.hip.put(r0), self.hip.put(r1), self.hip.put(np.zeros((n, 4), np.float32))
+
+    def trace(self, dev, sid):
+        rc = xa.lib().xt_trace_device_static(dev.handle, sid, xa.ACCEL_KDTREE, self.r0, self.r1, self.out, None, self.n)
+        assert rc == 0
+        return self.hip.get(self.out, np.zeros((self.n, 4), np.float32)).view(np.uint32)
+
+
+@pytest.fixture
+def rays():
+    r = Rays(4096, (-1, 1))
+    yield r
+    r.hip.free()
+
+
+def _resident_bytes(scene):
+    """Device memory of the scene walked on its kd-tree: what an upload needs at most."""
+    i = scene.info()
+    per_prim = 48 + 72 + 48 + (36 if i.any_vertex_normals else 0)  # FP32 and FP64 record, texture coordinates, normals
+    trees = 48 * i.n_oct_nodes + 4 * i.n_oct_refs + 8 * i.n_kd_nodes + (4 + 48) * i.n_kd_refs
+    return per_prim * i.n_prims + trees + (1 << 13)  # planes, materials, objects, rounding of the arrays
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,kw", [("strands", {"strands": 600}), ("icosphere", {"subdiv": 5}), ("terrain", {"n": 61})])
+def test_a_scene_that_fits_is_taken(device, rays, kind, kw):
+    """Every budget that holds the scene's arrays, its kd-tree and the copies of
+    the leaves takes it, whatever scratch the choice and the build of its index
+    could use with more; a released scene's memory is there for the next."""
+    scene = xa.Scene(scene_path(kind, **kw))
+    sid = device.upload(scene)
+    ref = rays.trace(device, sid)
+    device.release(sid)
+    assert (ref[:, 1] != xa.HIT_NONE).any()
+    need = _resident_bytes(scene)
+    for more in (1.0, 1.02, 1.1, 1.25, 1.5, 1.75, 2.0, 2.5, 3.0, 4.0, 6.0):
+        dev = xa.Device(0, hbm_budget=int(need * more))
+        for _ in range(2):
+            sid = dev.upload(scene)
+            hit = rays.trace(dev, sid)
+            assert np.array_equal(hit[:, 1], ref[:, 1])
+            np.testing.assert_allclose(hit[:, 0].view(np.float32), ref[:, 0].view(np.float32), rtol=1e-6)
+            dev.release(sid)
+        dev.close()
+    dev = xa.Device(0, hbm_budget=need // 2)
+    with pytest.raises(xa.XtError) as e:
+        dev.upload(scene)
+    assert e.value.code == E_BUDGET
+    dev.close()

@@ -425,6 +425,7 @@ int xt_scene_upload(xt_dev *d, const xt_scene *s, uint32_t *scene_id) {
     // primitives copied in leaf order (the object word replaced by the soup
     // index, so that a leaf's records are read without the reference list)
     if (!rc) rc = xt_bvh_build_into(d, ds, mem);
+    mem.release();  // what stays resident is not refused for the scratch
     if (!rc && !v.bvh) rc = xt_kd_leaf_copies(d, ds);
     if (rc) {
         (void)hipStreamSynchronize(d->stream);

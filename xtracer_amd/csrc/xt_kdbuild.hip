@@ -437,6 +437,7 @@ int xt_scene_build_kd_device(xt_dev *d, uint32_t scene_id, const xt_build_params
     xt_serve_forget_scene(d, scene_id);  // idle serving lanes hold the scene's old arrays
     XtScratch mem(d, xt_build_block(it->second.view.n_prims), false);
     int rc = xt_kd_build_into(d, it->second, p, mem);
+    mem.release();
     if (!rc && !it->second.view.bvh) rc = xt_kd_leaf_copies(d, it->second);
     if (rc) return rc;
     if (stats) *stats = it->second.kd_stats;

@@ -1,4 +1,4 @@
-"""Scenes at the limit of a device's HBM budget."""
+"""Scenes and tree builds at the limit of a device's HBM budget."""
 import numpy as np
 import pytest
 
@@ -66,3 +66,60 @@ def test_a_scene_that_fits_is_taken(device, rays, kind, kw):
         dev.upload(scene)
     assert e.value.code == E_BUDGET
     dev.close()
+def _uploads(scene, budget):
+    """Whether a device of this budget takes the scene."""
+    dev = xa.Device(0, hbm_budget=budget)
+    try:
+        dev.upload(scene)
+        return True
+    except xa.XtError as e:
+        assert e.code == E_BUDGET
+        return False
+    finally:
+        dev.close()
+
+
+def _least_budget(scene, hi, step=1 << 14):
+    lo = 0
+    assert _uploads(scene, hi)
+    while hi - lo > step:
+        mid = (lo + hi) // 2
+        lo, hi = (lo, mid) if _uploads(scene, mid) else (mid, hi)
+    return hi
+
+
+@pytest.mark.gpu
+def test_refused_rebuild_keeps_the_tree(rays):
+    """A rebuild that does not fit the budget leaves the resident tree, its
+    leaf copies and its hits as they were; one that fits replaces them."""
+    params = dict(kd_leaf_prims=1, kd_cost_intersect=60.0)
+    path = scene_path("strands", strands=600)
+    scene, finer = xa.Scene(path, threads=1), xa.Scene(path, threads=1, **params)
+    assert finer.info().n_kd_refs > scene.info().n_kd_refs
+    least = _least_budget(scene, 512 << 20)
+    outcomes = []
+    for k in range(25):
+        dev = xa.Device(0, hbm_budget=int(least * 1.25 ** k))
+        sid = dev.upload(scene)
+        nodes, refs, bounds, st = dev.kdtree(sid)
+        hits = rays.trace(dev, sid)
+        try:
+            dev.build_kd(sid, **params)
+            outcomes.append(True)
+            want = finer.kdtree()
+        except xa.XtError as e:
+            assert e.code == E_BUDGET
+            outcomes.append(False)
+            want = (nodes, refs, bounds)
+        got = dev.kdtree(sid)
+        for a, b in zip(got, want):
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+        assert np.array_equal(rays.trace(dev, sid)[:, 1], hits[:, 1])
+        # what the failed or finished build held is given back
+        dev.release(sid)
+        assert np.array_equal(rays.trace(dev, dev.upload(scene)), hits)
+        dev.close()
+        if outcomes[-3:] == [True] * 3:
+            break
+    assert not outcomes[0] and outcomes[-1]
+    assert outcomes == sorted(outcomes)

@@ -133,8 +133,9 @@ int xt_launch_trace_bufs(xt_dev *d, const DevScene &ds, int accel, const TraceBu
 class XtScratch;
 
 // Builds the kd-tree of a resident scene on the device (xt_kdbuild.hip) and
-// replaces the scene's kd arrays with it.
-int xt_kd_build_into(xt_dev *d, DevScene &ds, const xt_build_params *p, XtScratch &mem);
+// replaces the scene's kd arrays with it, with `leaf_copies` the copies of the
+// leaves' primitives among them. When that fails, the scene keeps its old ones.
+int xt_kd_build_into(xt_dev *d, DevScene &ds, const xt_build_params *p, bool leaf_copies, XtScratch &mem);
 // Builds the scene's wide BVH, unless its FP32 walk stays on the kd-tree
 // (view.bvh is null then). xt_bvhbuild.hip
 int xt_bvh_build_into(xt_dev *d, DevScene &ds, XtScratch &mem);

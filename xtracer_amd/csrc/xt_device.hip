@@ -419,7 +419,7 @@ int xt_scene_upload(xt_dev *d, const xt_scene *s, uint32_t *scene_id) {
     XtScratch mem(d, xt_build_block(v.n_prims), false);
     if (f.kd_deferred) {
         xt_build_params bp{f.kd_params.max_depth, f.kd_params.leaf_prims, f.kd_params.cost_intersect, 0, 0};
-        rc = xt_kd_build_into(d, ds, &bp, mem);
+        rc = xt_kd_build_into(d, ds, &bp, false, mem);
     }
     // the FP32 walk's index: the wide BVH, or the kd-tree with its leaves'
     // primitives copied in leaf order (the object word replaced by the soup

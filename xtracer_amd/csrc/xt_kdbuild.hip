@@ -94,7 +94,9 @@ const char *kdb_error(uint32_t e) {
 struct KdOut {
     XtKdNode *nodes = nullptr;
     uint32_t *refs = nullptr;
+    float4 *leaf = nullptr;    // copies of the leaves' primitives, or null
     uint64_t nodes_bytes = 0;  // with the references, which follow in the same block
+    uint64_t leaf_bytes = 0;
     float bounds[6] = {0, 0, 0, 0, 0, 0};
     xt_kd_build_stats stats{};
 };
@@ -111,11 +113,27 @@ int out_alloc(xt_dev *d, void **p, uint64_t bytes) {
 }
 
 void out_free(xt_dev *d, KdOut &o) {
-    if (o.nodes) {
-        (void)hipFree(o.nodes);
-        d->used -= std::min<uint64_t>(d->used, o.nodes_bytes);
-    }
+    for (auto pr : {std::make_pair((void *)o.nodes, o.nodes_bytes), std::make_pair((void *)o.leaf, o.leaf_bytes)})
+        if (pr.first) {
+            (void)hipFree(pr.first);
+            d->used -= std::min<uint64_t>(d->used, pr.second);
+        }
     o = KdOut();
+}
+
+// The primitives of n references, copied into the references' order.
+int copy_leaves(xt_dev *d, const SceneView &v, const uint32_t *refs, uint32_t n, float4 **leaf, uint64_t *bytes) {
+    const uint64_t b = std::max<uint64_t>(256, sizeof(XtPrim) * (uint64_t)n);
+    int rc = out_alloc(d, (void **)leaf, b);
+    if (rc) return rc;
+    *bytes = b;
+    if (n) {
+        hipLaunchKernelGGL(k_kdb_leaf_copies, dim3(grid_for(n, 256, 16384)), dim3(256), 0, d->stream, v.prims,
+                           v.n_prims, refs, n, *leaf);
+        XT_LAUNCHED();
+        XT_TRY(hipStreamSynchronize(d->stream));
+    }
+    return XT_OK;
 }
 
 int build(xt_dev *d, const SceneView &v, const xt_build_params *bp, XtScratch &mem, KdOut &o) {
@@ -373,7 +391,7 @@ void drop_kd(xt_dev *d, DevScene &ds) {
 
 }  // namespace
 
-int xt_kd_build_into(xt_dev *d, DevScene &ds, const xt_build_params *p, XtScratch &mem) {
+int xt_kd_build_into(xt_dev *d, DevScene &ds, const xt_build_params *p, bool leaf_copies, XtScratch &mem) {
     KdOut o;
     int rc = build(d, ds.view, p, mem, o);
     mem.reset();
@@ -382,14 +400,26 @@ int xt_kd_build_into(xt_dev *d, DevScene &ds, const xt_build_params *p, XtScratc
         XtScratch exact(d, 0, true);
         rc = build(d, ds.view, p, exact, o);
     }
-    if (rc) return rc;
-    XT_TRY(hipStreamSynchronize(d->stream));
+    if (!rc && leaf_copies) {
+        mem.release();
+        rc = copy_leaves(d, ds.view, o.refs, o.stats.n_refs, &o.leaf, &o.leaf_bytes);
+    }
+    if (!rc && hipStreamSynchronize(d->stream) != hipSuccess) {
+        d->err = "device kd-tree build: the stream failed";
+        rc = XT_E_DEVICE;
+    }
+    if (rc) {  // the scene keeps the tree it has
+        out_free(d, o);
+        return rc;
+    }
     drop_kd(d, ds);
     ds.allocs.push_back(o.nodes);
-    ds.kd_bytes = o.nodes_bytes;
+    if (o.leaf) ds.allocs.push_back(o.leaf);
+    ds.kd_bytes = o.nodes_bytes + o.leaf_bytes;
     ds.bytes += ds.kd_bytes;
     ds.view.kd = o.nodes;
     ds.view.kd_refs = o.refs;
+    ds.view.kd_leaf = o.leaf;
     for (int a = 0; a < 3; ++a) {
         ds.view.kb_lo[a] = o.bounds[a];
         ds.view.kb_hi[a] = o.bounds[3 + a];
@@ -401,21 +431,16 @@ int xt_kd_build_into(xt_dev *d, DevScene &ds, const xt_build_params *p, XtScratc
 }
 
 int xt_kd_leaf_copies(xt_dev *d, DevScene &ds) {
-    const uint64_t bytes = std::max<uint64_t>(256, sizeof(XtPrim) * (uint64_t)ds.n_kd_refs);
-    void *p = nullptr;
-    int rc = out_alloc(d, &p, bytes);
-    if (rc) return rc;
-    ds.allocs.push_back(p);
-    ds.bytes += bytes;
-    ds.kd_bytes += bytes;
-    ds.view.kd_leaf = (const float4 *)p;
-    if (ds.n_kd_refs) {
-        hipLaunchKernelGGL(k_kdb_leaf_copies, dim3(grid_for(ds.n_kd_refs, 256, 16384)), dim3(256), 0, d->stream,
-                           ds.view.prims, ds.view.n_prims, ds.view.kd_refs, ds.n_kd_refs, (float4 *)p);
-        XT_LAUNCHED();
-        XT_TRY(hipStreamSynchronize(d->stream));
+    float4 *leaf = nullptr;
+    uint64_t bytes = 0;
+    const int rc = copy_leaves(d, ds.view, ds.view.kd_refs, ds.n_kd_refs, &leaf, &bytes);
+    if (leaf) {
+        ds.allocs.push_back(leaf);
+        ds.bytes += bytes;
+        ds.kd_bytes += bytes;
     }
-    return XT_OK;
+    ds.view.kd_leaf = rc ? nullptr : leaf;
+    return rc;
 }
 
 extern "C" {
@@ -436,9 +461,7 @@ int xt_scene_build_kd_device(xt_dev *d, uint32_t scene_id, const xt_build_params
     XT_TRY(hipStreamSynchronize(d->stream));
     xt_serve_forget_scene(d, scene_id);  // idle serving lanes hold the scene's old arrays
     XtScratch mem(d, xt_build_block(it->second.view.n_prims), false);
-    int rc = xt_kd_build_into(d, it->second, p, mem);
-    mem.release();
-    if (!rc && !it->second.view.bvh) rc = xt_kd_leaf_copies(d, it->second);
+    const int rc = xt_kd_build_into(d, it->second, p, !it->second.view.bvh, mem);
     if (rc) return rc;
     if (stats) *stats = it->second.kd_stats;
     return XT_OK;

@@ -201,7 +201,11 @@ int xt_bvh_build_into(xt_dev *d, DevScene &ds, XtScratch &mem) {
             if (p) (void)hipFree(p);
         }
     } own;
-    XT_TRY(hipMalloc((void **)&own.p, bytes));
+    if (hipMalloc((void **)&own.p, bytes) != hipSuccess) {  // as beyond the budget: the kd-tree is walked
+        own.p = nullptr;
+        (void)hipGetLastError();
+        return XT_OK;
+    }
     uint32_t *const own_refs = (uint32_t *)(own.p + node_bytes);
     float4 *const own_leaf = (float4 *)(own.p + node_bytes + ref_bytes);
     XT_TRY(hipMemcpyAsync(own.p, wide, node_bytes, hipMemcpyDeviceToDevice, d->stream));

@@ -46,6 +46,7 @@ int dev_alloc(xt_dev *d, T **p, size_t count, std::vector<void *> *track, uint64
     hipError_t e = hipMalloc((void **)p, b);
     if (e != hipSuccess) {
         d->err = std::string("hipMalloc: ") + hipGetErrorString(e);
+        (void)hipGetLastError();  // not to be taken for a later launch's
         return XT_E_DEVICE;
     }
     d->used += b;

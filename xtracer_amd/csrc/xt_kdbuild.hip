@@ -107,7 +107,12 @@ int out_alloc(xt_dev *d, void **p, uint64_t bytes) {
         d->err = "device kd-tree exceeds the HBM budget";
         return XT_E_BUDGET;
     }
-    XT_TRY(hipMalloc(p, bytes));
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) {
+        d->err = std::string("hipMalloc: ") + hipGetErrorString(e);
+        (void)hipGetLastError();  // not to be taken for a later launch's
+        return XT_E_DEVICE;
+    }
     d->used += bytes;
     return XT_OK;
 }
@@ -341,7 +346,7 @@ int build(xt_dev *d, const SceneView &v, const xt_build_params *bp, XtScratch &m
     if (rc) {
         (void)hipStreamSynchronize(d->stream);
         out_free(d, o);
-        return rc;
+        return mem.exact ? rc : XT_E_BUDGET;  // it may fit beside less scratch
     }
     XT_TRY(hipMemcpyAsync(o.nodes + 1, &pad, sizeof pad, hipMemcpyHostToDevice, d->stream));
     for (const auto &lv : levels)

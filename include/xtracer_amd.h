@@ -154,7 +154,8 @@ typedef struct xt_kd_build_stats {
     double ms;                /* device time of the build (HIP events), 0 for a host-built tree */
     uint32_t n_nodes, n_refs; /* of the tree the scene holds */
     uint32_t depth, leaves, levels;
-    uint32_t pad;
+    uint32_t bvh_depth;       /* levels of the wide BVH that the scene's FP32 closest-hit walk uses; 0: it
+                                 walks the kd-tree */
 } xt_kd_build_stats;
 int xt_scene_build_kd_device(xt_dev *d, uint32_t scene_id, const xt_build_params *params, xt_kd_build_stats *stats);
 /* The resident kd-tree: n_nodes * 2 words, n_refs references, the root box

@@ -53,10 +53,10 @@ class BuildParams(ctypes.Structure):
 
 class KdBuildStats(ctypes.Structure):
     _fields_ = [("ms", ctypes.c_double)] + [(n, ctypes.c_uint32) for n in (
-        "n_nodes", "n_refs", "depth", "leaves", "levels", "pad")]
+        "n_nodes", "n_refs", "depth", "leaves", "levels", "bvh_depth")]
 
     def as_dict(self):
-        return {n: getattr(self, n) for n, _ in self._fields_ if n != "pad"}
+        return {n: getattr(self, n) for n, _ in self._fields_}
 
 
 class SceneInfo(ctypes.Structure):

@@ -218,7 +218,6 @@ int xt_bvh_build_into(xt_dev *d, DevScene &ds, XtScratch &mem) {
     ds.bytes += bytes;
     d->used += bytes;
     ds.bvh_depth = depth;
-    ds.n_bvh_nodes = base;
     v.bvh = (const uint4 *)own.p;
     v.bvh_refs = own_refs;
     v.bvh_leaf = own_leaf;

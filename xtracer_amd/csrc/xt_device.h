@@ -18,7 +18,7 @@ struct DevScene {
     uint64_t bytes = 0;
     uint64_t kd_bytes = 0;            // of the kd nodes, references and leaf copies (in `allocs`)
     uint32_t n_kd_nodes = 0, n_kd_refs = 0;
-    uint32_t n_bvh_nodes = 0, bvh_depth = 0;  // wide BVH (view.bvh), 0 without one
+    uint32_t bvh_depth = 0;           // levels of the wide BVH (view.bvh), 0 without one
     xt_kd_build_stats kd_stats{};     // of the last device build (zero for a host-built tree)
     bool pt_supported = true;
     bool materials_supported = true;

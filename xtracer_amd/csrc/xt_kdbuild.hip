@@ -468,7 +468,10 @@ int xt_scene_build_kd_device(xt_dev *d, uint32_t scene_id, const xt_build_params
     XtScratch mem(d, xt_build_block(it->second.view.n_prims), false);
     const int rc = xt_kd_build_into(d, it->second, p, !it->second.view.bvh, mem);
     if (rc) return rc;
-    if (stats) *stats = it->second.kd_stats;
+    if (stats) {
+        *stats = it->second.kd_stats;
+        stats->bvh_depth = it->second.bvh_depth;
+    }
     return XT_OK;
 }
 
@@ -493,6 +496,7 @@ int xt_scene_get_kd_device(xt_dev *d, uint32_t scene_id, uint32_t *nodes, uint32
         *stats = ds.kd_stats;
         stats->n_nodes = ds.n_kd_nodes;
         stats->n_refs = ds.n_kd_refs;
+        stats->bvh_depth = ds.bvh_depth;
     }
     return XT_OK;
 }

@@ -5,13 +5,17 @@
 // their hits are written and they get new rays. With whole groups of 64 rays
 // a wave ran as long as its longest ray: 10 of 64 lanes were active in the mean
 // instruction (1080p icosphere frame, rocprofv3), 26 with the refill. The
-// turn's phases end at 3 sixteenths of the working lanes: 4 and 6 were 1.6% and
-// 7% slower on the strands frame (23.2 ms).
+// turn's phases end at 3 sixteenths of the working lanes (strands frame at 2: the
+// same, at 4: 4% slower). What bounds a queue of about as many
+// rays as the card has lanes is each ray's chain of dependent loads, 27 records
+// of it on the strands: those of a leaf are loaded one ahead (50,000 strands,
+// 512x512x4 paths 6.70 to 6.05 ms, 1024x1024x8 20.0 to 18.4, 2 M random rays
+// 2.30 to 2.18; with whole groups of 64 rays and the same loads 6.2, 24.7, 3.0).
 #pragma once
 #include "xt_walk.h"
 
 #define XT_KD_KEEP 3      // sixteenths of the working lanes at which a phase ends
-#define XT_KD_WAVES 5     // waves per SIMD (96 VGPRs; at 6, with 88 B of spills, 3% slower)
+#define XT_KD_WAVES 5     // waves per SIMD (strands frame at 4: 3% slower, at 6: 10%, for spills)
 #define XT_KD_EPS 2e-6f   // relative widening of the walk's intervals
 
 // kd-tree walk with a ring of the STACK newest far children per lane in LDS
@@ -35,6 +39,7 @@ static __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(XT_KD
     bool more = true;
 
     const XtKdNode root = S.kd[0];
+    const float4 *const recs = S.kd_indexed ? S.prims : S.kd_leaf;
     bool alive = false, done = false, ok = true;
     uint32_t ri = 0, origin = XT_NONE;
     f3 o = mk(0, 0, 0), inv = mk(0, 0, 0);
@@ -147,23 +152,33 @@ static __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(XT_KD
         XtKdNode pre = root;
         if (alive && !node && count != lost) pre = S.kd[stk[off].x];
 
-        // leaf primitives
+        // leaf primitives, each record loaded while the one before it is
+        // tested (the empty asm ends the wait for a record before its test)
         bool leaf = alive && !node && payload != 0u;
+        float4 na = {}, nb = {}, nc = {};
+        uint32_t nrec = 0;
+        if (leaf) {
+            nrec = S.kd_indexed ? S.kd_refs[word >> 2] : word >> 2;
+            const float4 *rec = recs + 3 * (size_t)nrec;
+            na = rec[0];
+            nb = rec[1];
+            nc = rec[2];
+        }
         while (__popcll(__builtin_amdgcn_ballot_w64(leaf)) > keep) {
             if (leaf) {
-                uint32_t prim = word >> 2;
-                const float4 *rec;
-                if (S.kd_indexed) {
-                    prim = S.kd_refs[prim];
-                    rec = S.prims + 3 * (size_t)prim;
-                } else {
-                    rec = S.kd_leaf + 3 * (size_t)prim;
-                }
-                const float4 a = rec[0], b = rec[1], c = rec[2];
-                if (!S.kd_indexed) prim = __float_as_uint(b.w);
+                const float4 a = na, b = nb, c = nc;
+                const uint32_t prim = S.kd_indexed ? nrec : __float_as_uint(b.w);
                 word += 4u;
                 --payload;
                 leaf = payload != 0u;
+                if (leaf) {
+                    nrec = S.kd_indexed ? S.kd_refs[word >> 2] : word >> 2;
+                    const float4 *rec = recs + 3 * (size_t)nrec;
+                    na = rec[0];
+                    nb = rec[1];
+                    nc = rec[2];
+                }
+                asm volatile("" ::"v"(c.x), "v"(c.y), "v"(c.z), "v"(c.w));
                 if (prim != origin) {
                     if (XT_PRIM_TYPE(__float_as_uint(a.w)) == XT_PRIM_TRIANGLE) {
                         tri32_flat<false>(o, sx, sy, sz, kz, a, b, c, prim, best, inv, inv);

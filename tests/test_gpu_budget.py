@@ -41,7 +41,7 @@ def _resident_bytes(scene):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("kind,kw", [("strands", {"strands": 600}), ("icosphere", {"subdiv": 5}), ("terrain", {"n": 61})])
+@pytest.mark.parametrize("kind,kw", [("strands", {"strands": 600, "step": 0.4}), ("icosphere", {"subdiv": 5}), ("terrain", {"n": 61})])
 def test_a_scene_that_fits_is_taken(device, rays, kind, kw):
     """Every budget that holds the scene's arrays, its kd-tree and the copies of
     the leaves takes it, whatever scratch the choice and the build of its index
@@ -49,6 +49,7 @@ def test_a_scene_that_fits_is_taken(device, rays, kind, kw):
     scene = xa.Scene(scene_path(kind, **kw))
     sid = device.upload(scene)
     ref = rays.trace(device, sid)
+    assert (device.kdtree(sid)[3]["bvh_depth"] == 0) == (kind == "strands")  # both indexes are tried
     device.release(sid)
     assert (ref[:, 1] != xa.HIT_NONE).any()
     need = _resident_bytes(scene)
@@ -93,7 +94,7 @@ def test_refused_rebuild_keeps_the_tree(rays):
     """A rebuild that does not fit the budget leaves the resident tree, its
     leaf copies and its hits as they were; one that fits replaces them."""
     params = dict(kd_leaf_prims=1, kd_cost_intersect=60.0)
-    path = scene_path("strands", strands=600)
+    path = scene_path("strands", strands=600, step=0.4)
     scene, finer = xa.Scene(path, threads=1), xa.Scene(path, threads=1, **params)
     assert finer.info().n_kd_refs > scene.info().n_kd_refs
     least = _least_budget(scene, 512 << 20)
@@ -102,6 +103,7 @@ def test_refused_rebuild_keeps_the_tree(rays):
         dev = xa.Device(0, hbm_budget=int(least * 1.25 ** k))
         sid = dev.upload(scene)
         nodes, refs, bounds, st = dev.kdtree(sid)
+        assert st["bvh_depth"] == 0
         hits = rays.trace(dev, sid)
         try:
             dev.build_kd(sid, **params)

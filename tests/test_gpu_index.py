@@ -1,0 +1,172 @@
+"""Which index the FP32 walk of a scene uses: the wide BVH, at every depth that
+its kernels distinguish, or the kd-tree."""
+import numpy as np
+import pytest
+
+import xtracer_amd as xa
+from oracle.oracle import OracleScene
+from tests import scn
+from xtracer_amd import scenes
+from tests.helpers import scene_path, soup_to_object_local
+
+
+def _soup(tmp_path, tris):
+    scn.write_obj(tmp_path / "soup.obj", tris)
+    return xa.Scene(scn.write(tmp_path / "scene.scn", {"soup": dict(type="mesh", source="soup.obj")},
+                              {"soup": ("soup", "m")}, {"m": dict(type="lambert", kd=(0.5, 0.5, 0.5))}))
+
+
+def _depth(device, s):
+    sid = device.upload(s)
+    depth = device.kdtree(sid)[3]["bvh_depth"]
+    device.release(sid)
+    return depth
+
+
+def _check(device, s, o, d):
+    o, d = o.astype(np.float32), d.astype(np.float32)
+    sid = device.upload(s)
+    t, prim = device.trace(sid, o, d)[:2]
+    device.release(sid)
+    tr, obr, pr = OracleScene(s).trace(o.astype(np.float64), d.astype(np.float64))[:3]
+    obj, loc = soup_to_object_local(s.arrays(), prim)
+    same = (obj == obr) & ((obr < 0) | (loc == pr))
+    # FP32 misplaces an edge by up to 1e-4 of the triangles that these rays meet
+    assert same.mean() >= 0.999
+    hit = same & (obr >= 0)
+    assert hit.mean() > 0.25
+    np.testing.assert_allclose(t[hit], tr[hit], rtol=1e-5)
+    assert np.isinf(t[same & (obr < 0)]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 2, 4, 5, 8, 9, 33, 1023, 1024, 1025, 2500])
+def test_sparse_soups_walk_the_bvh(device, tmp_path, n):
+    """Around the sizes at which the build changes hands, against the oracle."""
+    rng = np.random.default_rng(n)
+    tris = rng.uniform(-2, 2, (n, 1, 3)) + rng.normal(scale=0.25 * n ** -0.5, size=(n, 3, 3))
+    s = _soup(tmp_path, tris)
+    depth = _depth(device, s)
+    assert depth > 0 and n <= 4 * 8 ** depth
+    o = rng.normal(size=(4000, 3))
+    o *= (9.0 / np.linalg.norm(o, axis=1))[:, None]
+    d = tris.mean(axis=1)[rng.integers(n, size=4000)] - o
+    d /= np.linalg.norm(d, axis=1)[:, None]
+    _check(device, s, o, d)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,scale", [(2500, 0.4), (20000, 0.2)])
+def test_crossing_soups_walk_the_kd_tree(device, tmp_path, n, scale):
+    rng = np.random.default_rng(n)
+    s = _soup(tmp_path, rng.uniform(-1, 1, (n, 1, 3)) + rng.normal(scale=scale, size=(n, 3, 3)))
+    assert _depth(device, s) == 0
+    o = rng.uniform(-1, 1, (4000, 3))
+    d = rng.normal(size=(4000, 3))
+    d /= np.linalg.norm(d, axis=1)[:, None]
+    _check(device, s, o, d)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ground", [0.0, 20.0])
+def test_a_floor_does_not_hide_dense_hair(device, tmp_path, ground):
+    """Crossing needles, alone and over a floor of 100 times their extent in area."""
+    rng = np.random.default_rng(1)
+    n = 30000
+    along, side = rng.normal(size=(2, n, 3))
+    along *= 0.3 / np.linalg.norm(along, axis=1)[:, None]
+    side *= 0.002 / np.linalg.norm(side, axis=1)[:, None]
+    mid = rng.uniform(-1, 1, (n, 3))
+    tris = np.stack([mid - along - side, mid - along + side, mid + along], 1)
+    if ground:
+        g = ground / 2
+        tris = np.concatenate([tris, [[[-g, -1, -g], [g, -1, -g], [g, -1, g]], [[-g, -1, -g], [g, -1, g], [-g, -1, g]]]])
+    assert _depth(device, _soup(tmp_path, tris)) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("away,bvh", [(0.0, True), (3e4, False)])
+def test_meshes_far_from_the_origin(device, tmp_path, away, bvh):
+    """The boxes' slack grows with the coordinates: a mesh whose triangles are
+    small against it is walked on the kd-tree."""
+    v, f = scenes.icosphere(6)
+    assert (_depth(device, _soup(tmp_path, v[f] + away)) > 0) == bvh
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_flat_boxes_walk_the_bvh(device, tmp_path, axis):
+    """Twelve layers of axis-aligned half cells, a sixth of them there: flat
+    boxes, and rays straight down on both halves of every cell."""
+    rng = np.random.default_rng(axis)
+    n, c = 24, 0.125
+    there = rng.random((12, n, n)) < 1 / 6
+    z, i, j = np.nonzero(there)
+    x, y, z = c * i - 1.5, c * j - 1.5, 0.25 * z - 1.5
+    tris = np.stack([np.stack([x, y, z], 1), np.stack([x + c, y, z], 1), np.stack([x + c, y + c, z], 1)], 1)
+    s = _soup(tmp_path, np.roll(tris, axis, axis=-1))
+    assert _depth(device, s) >= 3
+    u, v = [a.ravel() for a in np.meshgrid(c * np.arange(n) - 1.5, c * np.arange(n) - 1.5, indexing="ij")]
+    top = np.where(there.any(0), 5.0 + 1.5 - 0.25 * (11 - there[::-1].argmax(0)), np.inf).ravel()
+    sid = device.upload(s)
+    for du, dv, want in ((0.08, 0.04, top), (0.04, 0.08, np.full(n * n, np.inf))):
+        o = np.roll(np.stack([u + du, v + dv, np.full(u.size, 5.0)], 1), axis, axis=1)
+        d = np.roll(np.tile([0.0, 0.0, -1.0], (u.size, 1)), axis, axis=1)
+        t = device.trace(sid, o.astype(np.float32), d.astype(np.float32))[0]
+        np.testing.assert_allclose(t, want, rtol=1e-6)
+    device.release(sid)
+    o = rng.normal(size=(4000, 3))
+    o *= (9.0 / np.linalg.norm(o, axis=1))[:, None]
+    d = np.roll(tris, axis, axis=-1).mean(axis=1)[rng.integers(len(tris), size=4000)] - o
+    _check(device, s, o, d / np.linalg.norm(d, axis=1)[:, None])
+
+
+@pytest.mark.gpu
+def test_equal_primitives_walk_the_bvh(device, tmp_path):
+    """Each triangle three times over: the tie goes to the first, as in the oracle."""
+    rng = np.random.default_rng(2)
+    tris = np.tile(rng.uniform(-2, 2, (400, 1, 3)) + rng.normal(scale=0.02, size=(400, 3, 3)), (3, 1, 1))
+    s = _soup(tmp_path, tris)
+    assert _depth(device, s) >= 3
+    o = rng.normal(size=(4000, 3))
+    o *= (9.0 / np.linalg.norm(o, axis=1))[:, None]
+    d = tris.mean(axis=1)[rng.integers(1200, size=4000)] - o
+    d /= np.linalg.norm(d, axis=1)[:, None]
+    _check(device, s, o, d)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,kw,bvh", [("spheres", {}, True), ("icosphere", {"subdiv": 5}, True),
+                                         ("terrain", {"n": 41}, True), ("strands", {"strands": 600}, True),
+                                         ("strands", {"strands": 600, "step": 0.4}, False)])
+def test_scenes(device, kind, kw, bvh):
+    assert (_depth(device, xa.Scene(scene_path(kind, **kw))) > 0) == bvh
+
+
+def _shells(n, per=30):
+    """Shells of large triangles, each twice as large as the next and around it:
+    a ray through the middle meets parts of every one, with the rest of the
+    tree among their siblings."""
+    rng = np.random.default_rng(n)
+    size = np.repeat(1e4 * 0.5 ** np.arange(n), per)
+    d = rng.normal(size=(n * per, 1, 3))
+    c = d / np.linalg.norm(d, axis=2, keepdims=True)
+    return size[:, None, None] * (c + rng.normal(scale=0.25, size=(n * per, 3, 3)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,least,most", [(8, 1, 10), (10, 1, 10), (14, 11, 14), (16, 15, 18), (24, 19, 24), (28, 0, 0)])
+def test_deep_trees(device, tmp_path, n, least, most):
+    """Trees of up to 10, 14 and 24 levels (the trace kernels' stacks of 8, 12
+    and 24 entries) and one that is too deep for any, against the oracle."""
+    s = _soup(tmp_path, _shells(n))
+    sid = device.upload(s)
+    assert least <= device.kdtree(sid)[3]["bvh_depth"] <= most
+    rng = np.random.default_rng(7)
+    size = 1e4 * 0.5 ** rng.integers(0, n - 5, 4000)
+    o, aim = rng.normal(size=(2, 4000, 3))
+    o *= (2.5 * size / np.linalg.norm(o, axis=1))[:, None]
+    d = 0.1 * size[:, None] * aim - o
+    d /= np.linalg.norm(d, axis=1)[:, None]
+    device.release(sid)
+    _check(device, s, o, d)

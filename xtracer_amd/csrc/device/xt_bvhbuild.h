@@ -26,6 +26,14 @@ struct BvbCtl {
     uint32_t m, next;  // clusters, next binary node
 };
 
+// What a build reports to the host.
+struct BvbInfo {
+    uint32_t bad, root;  // whether a box is not finite; binary node of the root, or XT_NONE
+    // of a sample of rays: wide nodes visited and primitives tested on the
+    // BVH, leaves visited and primitives tested on the kd-tree
+    unsigned long long nodes, bvh_tests, leaves, kd_tests;
+};
+
 __device__ __forceinline__ float bvb_area(const float lo[3], const float hi[3]) {
     const float x = hi[0] - lo[0], y = hi[1] - lo[1], z = hi[2] - lo[2];
     return x * y + y * z + z * x;
@@ -61,47 +69,15 @@ __device__ __forceinline__ void bvb_prim_box(const float4 *prims, uint32_t p, fl
     }
 }
 
-// Per block: the sum of the primitives' box half areas, of the triangles'
-// areas (a sphere counts as a quarter of its box, half its surface's share)
-// and the number of boxes that are not finite.
-static __global__ __launch_bounds__(256) void k_bvb_stats(const float4 *prims, uint32_t n, double *part) {
-    __shared__ double s[3][256];
-    double box = 0, tri = 0, bad = 0;
-    for (uint32_t p = blockIdx.x * 256 + threadIdx.x; p < n; p += gridDim.x * 256) {
-        float lo[3], hi[3];
-        bvb_prim_box(prims, p, lo, hi);
-        const float ha = bvb_area(lo, hi);
-        if (!(fabsf(ha) < 1e30f) || !(fabsf(lo[0]) < 1e30f) || !(fabsf(lo[1]) < 1e30f) || !(fabsf(lo[2]) < 1e30f)) {
-            bad += 1;
-            continue;
-        }
-        box += ha;
-        const float4 a = prims[3 * (size_t)p], b = prims[3 * (size_t)p + 1], c = prims[3 * (size_t)p + 2];
-        if (XT_PRIM_TYPE(__float_as_uint(a.w)) == XT_PRIM_TRIANGLE) {
-            const f3 x = cross3(sub(mk(b.x, b.y, b.z), mk(a.x, a.y, a.z)), sub(mk(c.x, c.y, c.z), mk(a.x, a.y, a.z)));
-            tri += 0.5 * sqrt((double)dot3(x, x));
-        } else {
-            tri += 0.25 * ha;
-        }
-    }
-    s[0][threadIdx.x] = box;
-    s[1][threadIdx.x] = tri;
-    s[2][threadIdx.x] = bad;
-    __syncthreads();
-    for (uint32_t o = 128; o > 0; o >>= 1) {
-        if (threadIdx.x < o)
-            for (int k = 0; k < 3; ++k) s[k][threadIdx.x] += s[k][threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x < 3) part[3 * blockIdx.x + threadIdx.x] = s[threadIdx.x][0];
-}
-
 static __global__ __launch_bounds__(256) void k_bvb_keys(const float4 *prims, uint32_t n, float3 org, float scale,
-                                                         uint64_t *key, uint32_t *val) {
+                                                         uint64_t *key, uint32_t *val, BvbInfo *info) {
     const uint32_t p = blockIdx.x * 256 + threadIdx.x;
     if (p >= n) return;
     float lo[3], hi[3];
     bvb_prim_box(prims, p, lo, hi);
+    const float ha = bvb_area(lo, hi);
+    if (!(fabsf(ha) < 1e30f) || !(fabsf(lo[0]) < 1e30f) || !(fabsf(lo[1]) < 1e30f) || !(fabsf(lo[2]) < 1e30f))
+        info->bad = 1;
     const float og[3] = {org.x, org.y, org.z};
     uint64_t k = 0;
     for (int a = 0; a < 3; ++a) {
@@ -580,4 +556,112 @@ static __global__ __launch_bounds__(256) void k_bvb_records(const float4 *prims,
         leaf[3 * (size_t)i + 1] = b;
         leaf[3 * (size_t)i + 2] = prims[3 * (size_t)p + 2];
     }
+}
+
+// ------------------------------------------------------------------- the choice
+
+// Ray i of the sample: through or from a primitive drawn by i, in a random
+// direction; even rays come from outside the scene, odd ones leave the
+// primitive as a bounce ray does.
+__device__ __forceinline__ RayF probe_ray(const SceneView &S, uint32_t i) {
+    const uint32_t key = xt_stream(xt_mix32(i + 1u), 1u);
+    const uint32_t p = xt_draw(key, 0) % S.n_prims;
+    const float4 a = S.prims[3 * (size_t)p], b = S.prims[3 * (size_t)p + 1], c = S.prims[3 * (size_t)p + 2];
+    const float z = 2.f * xt_unit32(xt_draw(key, 1)) - 1.f, phi = 6.2831853f * xt_unit32(xt_draw(key, 2));
+    const float s = sqrtf(fmaxf(0.f, 1.f - z * z));
+    RayF r;
+    r.d = mk(s * cosf(phi), s * sinf(phi), z);
+    f3 at;
+    if (XT_PRIM_TYPE(__float_as_uint(a.w)) == XT_PRIM_TRIANGLE)
+        at = mk((a.x + b.x + c.x) / 3.f, (a.y + b.y + c.y) / 3.f, (a.z + b.z + c.z) / 3.f);
+    else at = add(mk(a.x, a.y, a.z), scl(r.d, fabsf(b.x)));
+    r.origin = XT_NONE;
+    r.self_t = 0.f;
+    if (i & 1u) {
+        r.o = at;
+        r.origin = p;
+    } else {
+        const f3 ext = mk(S.kb_hi[0] - S.kb_lo[0], S.kb_hi[1] - S.kb_lo[1], S.kb_hi[2] - S.kb_lo[2]);
+        r.o = sub(at, scl(r.d, sqrtf(dot3(ext, ext))));
+    }
+    return r;
+}
+
+struct ProbeTester {
+    Tester32 t;
+    uint32_t leaves, tests;
+    __device__ __forceinline__ float limit() const { return t.limit(); }
+    __device__ __forceinline__ void test_leaf_range(uint32_t k, uint32_t n) {
+        ++leaves;
+        tests += n;
+        for (uint32_t j = 0; j < n; ++j) t.test(t.S.kd_refs[k + j]);
+    }
+};
+
+__device__ __forceinline__ void probe_add(unsigned long long *to, uint32_t v) {
+    for (int o = 32; o > 0; o >>= 1) v += (uint32_t)__shfl_xor((int)v, o);
+    if (lane_id() == 0) atomicAdd(to, (unsigned long long)v);
+}
+
+// Walks the sample on both indexes, one lane a ray, and adds up the steps: the
+// first half of the blocks on the kd-tree, the second half the same rays on the
+// BVH. Bound by the longest chain of dependent loads: one wave on every compute
+// unit.
+static __global__ __launch_bounds__(64) void k_bvb_probe(const SceneView S, BvbInfo *out) {
+    __shared__ uint2 kstk[(XT_KD_STACK + 1) * 64];
+    __shared__ uint32_t bstk[24 * 64];
+    const uint32_t half = gridDim.x / 2;
+    const RayF r = probe_ray(S, (blockIdx.x % half) * 64 + threadIdx.x);
+    Tester32 tst{S, r, tsmall_of(r.o), {}, make_shear(r.d)};
+    seed_best(r, tst.best);
+    for (uint32_t k = 0; k < S.n_planes; ++k)
+        plane32(r.o, r.d, tst.tsmall, S.planes[k], XT_PLANE_BASE + k, tst.best);
+    if (blockIdx.x < half) {
+        ProbeTester kd{tst, 0, 0};
+        (void)walk_kd<XT_KD_STACK>(S, kd, r.o, r.d, kstk + threadIdx.x, 64, 1e-6f);
+        probe_add(&out->leaves, kd.leaves);
+        probe_add(&out->kd_tests, kd.tests);
+        return;
+    }
+
+    // the walk of k_trace_bvh, one lane a ray
+    const f3 inv = mk(rcp_dir(r.d.x), rcp_dir(r.d.y), rcp_dir(r.d.z));
+    const f3 eta = box_slack(r.o, inv, coord_max(S));
+    const uint32_t oct = octant_of(inv);
+    uint32_t grp = 1u << oct, sp = threadIdx.x, nodes = 0, tests = 0;
+    while (grp) {
+        const uint32_t bit = (uint32_t)__builtin_ctz(grp);
+        grp &= grp - 1u;
+        const uint4 *nd = S.bvh + 8 * (size_t)((grp >> 8) + (bit ^ oct));
+        const half8 *pl = (const half8 *)(nd + 2);
+        const uint4 n1 = nd[1];
+        ++nodes;
+        const uint32_t nx = oct & 1u ? 3u : 0u, ny = oct & 2u ? 4u : 1u, nz = oct & 4u ? 5u : 2u;
+        const uint32_t hits = wide_hits(*(const float4 *)nd, pl[nx], pl[ny], pl[nz], pl[3u - nx], pl[5u - ny],
+                                        pl[7u - nz], r.o, inv, eta, tst.limit() * (1.f + 4e-6f));
+        for (uint32_t lh = hits & n1.z & 0xffu; lh; lh &= lh - 1u) {
+            const uint32_t slot = (uint32_t)__builtin_ctz(lh);
+            const uint32_t below = n1.z & ((1u << slot) - 1u) * 0x010101u, cb = n1.z >> slot;
+            const uint32_t k0 = n1.y + (uint32_t)__popc(below) + (uint32_t)__popc(below >> 16);
+            const uint32_t n = 1u + ((cb >> 8) & 1u) + ((cb >> 15) & 2u);
+            tests += n;
+            for (uint32_t k = k0; k < k0 + n; ++k) tst.test(S.bvh_refs[k]);
+        }
+        const uint32_t ih = octant_order(hits & (n1.z >> 24), oct);
+        if (ih) {
+            if (grp & 0xffu) {
+                bstk[sp] = grp;
+                sp += 64;
+            }
+            grp = ih | n1.x << 8;
+        } else if (!(grp & 0xffu)) {
+            grp = 0;
+            if (sp >= 64) {
+                sp -= 64;
+                grp = bstk[sp];
+            }
+        }
+    }
+    probe_add(&out->nodes, nodes);
+    probe_add(&out->bvh_tests, tests);
 }

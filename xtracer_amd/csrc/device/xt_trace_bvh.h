@@ -93,6 +93,47 @@ __device__ __forceinline__ float lane_value(float v, int l) {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 
+// The slots of a node whose boxes the ray enters before lim: n0 the grid's
+// origin and step, near and far planes by the ray's signs.
+__device__ __forceinline__ uint32_t wide_hits(const float4 n0, half8 qnx, half8 qny, half8 qnz, half8 qfx, half8 qfy,
+                                              half8 qfz, f3 o, f3 inv, f3 eta, float lim) {
+    const float dx = n0.w * inv.x, dy = n0.w * inv.y, dz = n0.w * inv.z;
+    const float px = n0.x - o.x, py = n0.y - o.y, pz = n0.z - o.z;
+    const float anx = px * inv.x - eta.x, afx = px * inv.x + eta.x;
+    const float any_ = py * inv.y - eta.y, afy = py * inv.y + eta.y;
+    const float anz = pz * inv.z - eta.z, afz = pz * inv.z + eta.z;
+    uint32_t hits = 0;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        const float t0 = fmaxf(fmaxf(fmaxf((float)qnx[c] * dx + anx, (float)qny[c] * dy + any_),
+                                     (float)qnz[c] * dz + anz), 0.f);
+        const float t1 = fminf(fminf(fminf((float)qfx[c] * dx + afx, (float)qfy[c] * dy + afy),
+                                     (float)qfz[c] * dz + afz), lim);
+        hits |= t0 <= t1 ? 1u << c : 0u;
+    }
+    return hits;
+}
+
+// Slot order to octant order: bit s to bit s ^ oct.
+__device__ __forceinline__ uint32_t octant_order(uint32_t ih, uint32_t oct) {
+    ih = (oct & 1u) ? ((ih << 1) & 0xaau) | ((ih >> 1) & 0x55u) : ih;
+    ih = (oct & 2u) ? ((ih << 2) & 0xccu) | ((ih >> 2) & 0x33u) : ih;
+    return (oct & 4u) ? ((ih << 4) & 0xf0u) | (ih >> 4) : ih;
+}
+
+// Sign bits of a direction, and by how much the walk widens boxes for it.
+__device__ __forceinline__ uint32_t octant_of(f3 inv) {
+    return (inv.x < 0.f ? 1u : 0u) | (inv.y < 0.f ? 2u : 0u) | (inv.z < 0.f ? 4u : 0u);
+}
+__device__ __forceinline__ float coord_max(const SceneView &S) {
+    return fmaxf(fmaxf(fmaxf(fabsf(S.kb_lo[0]), fabsf(S.kb_hi[0])), fmaxf(fabsf(S.kb_lo[1]), fabsf(S.kb_hi[1]))),
+                 fmaxf(fabsf(S.kb_lo[2]), fabsf(S.kb_hi[2])));
+}
+__device__ __forceinline__ f3 box_slack(f3 o, f3 inv, float smax) {
+    const float e = XT_W_SLACK * (fmaxf(fabsf(o.x), fmaxf(fabsf(o.y), fabsf(o.z))) + smax);
+    return mk(e * fabsf(inv.x), e * fabsf(inv.y), e * fabsf(inv.z));
+}
+
 // STACK: the deepest a walk's stack gets, which the tree's depth bounds. A
 // stack entry is the rest of a group of siblings: the hits not yet visited in
 // octant order (bits 0-7) and the node of slot 0 (bits 8-31).
@@ -115,9 +156,7 @@ static __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(XT_W_
     RaySource R;
     source_init(R, n, waves, T);
     bool more = true;
-    const float smax = fmaxf(fmaxf(fmaxf(fabsf(S.kb_lo[0]), fabsf(S.kb_hi[0])),
-                                   fmaxf(fabsf(S.kb_lo[1]), fabsf(S.kb_hi[1]))),
-                             fmaxf(fabsf(S.kb_lo[2]), fabsf(S.kb_hi[2])));
+    const float smax = coord_max(S);
 
     bool alive = false, done = false;
     uint32_t ri = 0, origin = XT_NONE, oct = 0, kz = 0;
@@ -212,9 +251,8 @@ static __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(XT_W_
                                 plane32(r.o, r.d, tsmall, S.planes[k], XT_PLANE_BASE + k, best);
                         const float dk = ray_shear(r.d, kz, sx, sy, sz);
                         inv = mk(rcp_dir(r.d.x), rcp_dir(r.d.y), rcp_dir(r.d.z));
-                        const float e = XT_W_SLACK * (fmaxf(fabsf(o.x), fmaxf(fabsf(o.y), fabsf(o.z))) + smax);
-                        eta = mk(e * fabsf(inv.x), e * fabsf(inv.y), e * fabsf(inv.z));
-                        oct = (inv.x < 0.f ? 1u : 0u) | (inv.y < 0.f ? 2u : 0u) | (inv.z < 0.f ? 4u : 0u);
+                        eta = box_slack(o, inv, smax);
+                        oct = octant_of(inv);
                         // the root as the only hit of a group above it
                         grp = 1u << oct;
                         lhit = tn = 0;
@@ -321,29 +359,12 @@ static __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(XT_W_
                 const half8 qnx = *(const half8 *)(nd + (offx ^ sw)), qfx = *(const half8 *)(nd + ((112u - offx) ^ sw));
                 const half8 qny = *(const half8 *)(nd + (offy ^ sw)), qfy = *(const half8 *)(nd + ((144u - offy) ^ sw));
                 const half8 qnz = *(const half8 *)(nd + (offz ^ sw)), qfz = *(const half8 *)(nd + ((176u - offz) ^ sw));
-                const float dx = n0.w * inv.x, dy = n0.w * inv.y, dz = n0.w * inv.z;
-                const float px = n0.x - o.x, py = n0.y - o.y, pz = n0.z - o.z;
-                const float anx = px * inv.x - eta.x, afx = px * inv.x + eta.x;
-                const float any_ = py * inv.y - eta.y, afy = py * inv.y + eta.y;
-                const float anz = pz * inv.z - eta.z, afz = pz * inv.z + eta.z;
-                const float lim = fminf(best.t, shared_t) * (1.f + 4e-6f);
-                uint32_t hits = 0;
-#pragma unroll
-                for (int c = 0; c < 8; ++c) {
-                    const float t0 = fmaxf(fmaxf(fmaxf((float)qnx[c] * dx + anx, (float)qny[c] * dy + any_),
-                                                 (float)qnz[c] * dz + anz), 0.f);
-                    const float t1 = fminf(fminf(fminf((float)qfx[c] * dx + afx, (float)qfy[c] * dy + afy),
-                                                 (float)qfz[c] * dz + afz), lim);
-                    hits |= t0 <= t1 ? 1u << c : 0u;
-                }
+                const uint32_t hits = wide_hits(n0, qnx, qny, qnz, qfx, qfy, qfz, o, inv, eta,
+                                                fminf(best.t, shared_t) * (1.f + 4e-6f));
                 lmask = n1.z;
                 lhit = hits & lmask & 0xffu;
                 tbase = n1.y;
-                uint32_t ih = hits & (lmask >> 24);
-                // slot order to octant order
-                ih = (oct & 1u) ? ((ih << 1) & 0xaau) | ((ih >> 1) & 0x55u) : ih;
-                ih = (oct & 2u) ? ((ih << 2) & 0xccu) | ((ih >> 2) & 0x33u) : ih;
-                ih = (oct & 4u) ? ((ih << 4) & 0xf0u) | (ih >> 4) : ih;
+                const uint32_t ih = octant_order(hits & (lmask >> 24), oct);
                 if (ih) {
                     if (grp & 0xffu) {
                         stk[sp] = grp;

@@ -1,9 +1,10 @@
 // Device build of a resident scene's wide BVH, the index of the FP32
 // closest-hit walk: primitives sorted by Morton code, neighbouring clusters
 // merged pairwise to a binary tree, that tree cut into 8-wide nodes and leaves
-// of up to 4 primitives at the least expected cost, and the nodes written level
-// by level. Launches and read-backs bound it for small scenes, memory for large ones
-// (about 320 bytes of scratch a primitive).
+// of up to 4 primitives at the least expected cost, the nodes written level
+// by level; then a sample of rays chooses between it and the kd-tree. Launches
+// and read-backs bound it for small scenes, memory for large ones (364 bytes of
+// scratch a primitive).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -36,7 +37,7 @@
 
 namespace {
 
-constexpr uint32_t kStatBlocks = 256;
+constexpr uint32_t kProbeBlocks = 128;  // of 64 sample rays
 constexpr int kMaxRounds = 160;   // of pairwise merging; a scene that needs more keeps the kd-tree walk
 constexpr uint32_t kMaxDepth = 24;  // the deepest stack of the trace kernel
 
@@ -61,9 +62,33 @@ int scan(xt_dev *d, const uint64_t *in, uint64_t *out, uint32_t n, uint64_t *til
     return XT_OK;
 }
 
+// Which index the FP32 walk of a scene takes, from what a sample of rays costs
+// on each (k_bvb_probe). The kd-tree clips primitives and ends a ray at its
+// first hit; the wide BVH is cheaper for each ray until many boxes overlap at
+// one place: fields of crossing triangles, dense hair, meshes so far from the
+// origin that the boxes' slack is large against their triangles. No figure of the
+// primitives alone told these apart (the boxes' area over the primitives' is 3.4
+// for meshes, 5 for every soup below, 8 to 230 for hair, and one large floor
+// hides a scene of hair from it). The weights are fitted to frames of 512x512x4
+// and 1024x1024x4 paths and 1 M random rays of 57 scenes; one of them (300 random
+// triangles) goes to a walk that is more than 2% slower than the other, by 12%. Time on the
+// BVH over time on the kd-tree (geometric mean), and the ratio of the two costs:
+//   icosphere of 1.31 M triangles 0.41 (0.37), one of 0.33 M 3,000 radii from
+//     the origin 0.99 (0.88), 10,000 radii 1.95 (3.1)
+//   terrain 0.57 (0.37), 64 spheres 0.86 (0.55), 500 random boxes 1.02 (1.2)
+//   1 M random triangles in a cube 700 times as wide 0.48 (0.37), 200 times 0.98
+//     (0.88), 70 times 2.3 (3.1), 20 times 6.7 (15)
+//   strands: 2,000 0.65 (0.50), 10,000 0.81 (0.82), 30,000 1.21 (1.50), 50,000
+//     1.61 (2.31), these over a floor of two triangles 1.57 (2.22)
+bool bvh_walk_is_cheaper(const BvbInfo &s, uint32_t rays) {
+    const double bvh = (double)s.nodes + 0.8 * (double)s.bvh_tests + 2.0 * rays;
+    const double kd = 4.0 * (double)s.leaves + 0.5 * (double)s.kd_tests;
+    return bvh <= kd;
+}
+
 }  // namespace
 
-// Builds the wide BVH of a resident scene whose primitives and kd-tree bounds
+// Builds the wide BVH of a resident scene whose primitives, kd-tree and bounds
 // are in place, if the trace would rather walk it than the kd-tree: `view`
 // then names its arrays, which join ds.allocs. Otherwise view.bvh stays null.
 int xt_bvh_build_into(xt_dev *d, DevScene &ds, XtScratch &mem) {
@@ -78,15 +103,15 @@ int xt_bvh_build_into(xt_dev *d, DevScene &ds, XtScratch &mem) {
     const size_t scan_n = std::max<size_t>((size_t)n + 4096, 256ull * sort_tiles) + 1;
     const uint32_t scan_tiles = (uint32_t)((scan_n + XT_KDB_TILE) / XT_KDB_TILE) + 1;
     const uint32_t cap = n + 4096;  // wide nodes, the unused ones among siblings included
-    const size_t caps[] = {3 * kStatBlocks * sizeof(double), 8ull * n, 8ull * n, 4ull * cap, 4ull * cap,
+    const size_t caps[] = {sizeof(BvbInfo), 8ull * n, 8ull * n, 4ull * cap, 4ull * cap,
                            2ull * n * sizeof(BvbNode), 4ull * n, 8ull * scan_n, 8ull * scan_n, 8ull * scan_tiles,
-                           32ull * cap, (size_t)cap * sizeof(XtWideNode), 2 * sizeof(BvbCtl), 4};
+                           32ull * cap, (size_t)cap * sizeof(XtWideNode), 2 * sizeof(BvbCtl)};
     Block B;
     for (size_t c : caps) B.bytes += (c + 255) & ~(size_t)255;
     int rc = mem.take((void **)&B.p, B.bytes);
     if (rc == XT_E_BUDGET) return XT_OK;
     if (rc) return rc;
-    double *part = B.take<double>(3 * kStatBlocks);
+    BvbInfo *info = B.take<BvbInfo>(1);
     uint64_t *key[2] = {B.take<uint64_t>(n), nullptr};
     key[1] = B.take<uint64_t>(n);
     uint32_t *val[2] = {B.take<uint32_t>(cap), nullptr};
@@ -98,27 +123,15 @@ int xt_bvh_build_into(xt_dev *d, DevScene &ds, XtScratch &mem) {
     uint32_t *children = B.take<uint32_t>(8ull * cap);
     XtWideNode *wide = B.take<XtWideNode>(cap);
     BvbCtl *ctl = B.take<BvbCtl>(2);
-    uint32_t *root = B.take<uint32_t>(1);
 
-    hipLaunchKernelGGL(k_bvb_stats, dim3(kStatBlocks), dim3(256), 0, d->stream, v.prims, n, part);
-    XT_LAUNCHED();
-    XT_TRY(hipMemcpyAsync(d->host_words, part, 3 * kStatBlocks * sizeof(double), hipMemcpyDeviceToHost, d->stream));
-    XT_TRY(hipStreamSynchronize(d->stream));
-    double box = 0, tri = 0, bad = 0;
-    for (uint32_t k = 0; k < kStatBlocks; ++k) {
-        box += ((const double *)d->host_words)[3 * k];
-        tri += ((const double *)d->host_words)[3 * k + 1];
-        bad += ((const double *)d->host_words)[3 * k + 2];
-    }
-    if (bad > 0 || !(box <= XT_BVH_MAX_BOX_RATIO * tri)) return XT_OK;
-
+    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, d->stream, (uint32_t *)info, 0u, sizeof(BvbInfo) / 4);
     // Morton order
     float ext = 0.f;
     for (int a = 0; a < 3; ++a) ext = std::max(ext, v.kb_hi[a] - v.kb_lo[a]);
     const float scale = ext > 0.f ? 2097152.f / ext : 0.f;
     const unsigned nb = (n + 255) / 256;
     hipLaunchKernelGGL(k_bvb_keys, dim3(nb), dim3(256), 0, d->stream, v.prims, n,
-                       make_float3(v.kb_lo[0], v.kb_lo[1], v.kb_lo[2]), scale, key[0], val[0]);
+                       make_float3(v.kb_lo[0], v.kb_lo[1], v.kb_lo[2]), scale, key[0], val[0], info);
     for (uint32_t pass = 0; pass < 8; ++pass) {
         const int a = (int)(pass & 1u);
         hipLaunchKernelGGL(k_bvb_count, dim3(sort_tiles), dim3(256), 0, d->stream, (const uint64_t *)key[a], n,
@@ -155,15 +168,16 @@ int xt_bvh_build_into(xt_dev *d, DevScene &ds, XtScratch &mem) {
         }
     }
     hipLaunchKernelGGL(k_bvb_small, dim3(1), dim3(XT_BVB_SMALL), 0, d->stream, nodes, 2u * n,
-                       (const uint32_t *)val[c], (const BvbCtl *)(ctl + q), root);
+                       (const uint32_t *)val[c], (const BvbCtl *)(ctl + q), &info->root);
     XT_LAUNCHED();
-    XT_TRY(hipMemcpyAsync(d->host_words, root, 4, hipMemcpyDeviceToHost, d->stream));
+    const BvbInfo *const host = (const BvbInfo *)d->host_words;
+    XT_TRY(hipMemcpyAsync(d->host_words, info, sizeof(BvbInfo), hipMemcpyDeviceToHost, d->stream));
     XT_TRY(hipStreamSynchronize(d->stream));
-    if (((const uint32_t *)d->host_words)[0] >= 2u * n) return XT_OK;  // not merged to one root
+    if (host->bad || host->root >= 2u * n) return XT_OK;  // boxes that are not finite, or not merged to one root
 
     // wide nodes, level by level
     uint32_t *items[2] = {val[0], val[1]}, *refs = nn;
-    XT_TRY(hipMemcpyAsync(items[0], root, 4, hipMemcpyDeviceToDevice, d->stream));
+    XT_TRY(hipMemcpyAsync(items[0], &info->root, 4, hipMemcpyDeviceToDevice, d->stream));
     uint32_t base = 0, prim_base = 0, count = 1, depth = 0;
     for (int a = 0; count > 0; a ^= 1) {
         if (++depth > kMaxDepth || (uint64_t)base + count > std::min(cap, XT_WIDE_MAX_NODES)) return XT_OK;
@@ -191,7 +205,13 @@ int xt_bvh_build_into(xt_dev *d, DevScene &ds, XtScratch &mem) {
         d->err = "wide BVH build: primitives missing";
         return XT_E_STATE;
     }
-    // the scene's own arrays
+    SceneView w = v;
+    w.bvh = (const uint4 *)wide;
+    w.bvh_refs = refs;
+    hipLaunchKernelGGL(k_bvb_probe, dim3(2 * kProbeBlocks), dim3(64), 0, d->stream, w, info);
+    XT_LAUNCHED();
+    XT_TRY(hipMemcpyAsync(d->host_words, info, sizeof(BvbInfo), hipMemcpyDeviceToHost, d->stream));
+    // the scene's own arrays, allocated while the sample is walked
     const uint64_t node_bytes = (uint64_t)base * sizeof(XtWideNode), ref_bytes = (4ull * n + 255) & ~255ull;
     const uint64_t bytes = node_bytes + ref_bytes + 48ull * n;
     if (d->budget && d->used + bytes > d->budget) return XT_OK;
@@ -214,6 +234,7 @@ int xt_bvh_build_into(xt_dev *d, DevScene &ds, XtScratch &mem) {
                        (const uint32_t *)refs, n, own_leaf);
     XT_LAUNCHED();
     XT_TRY(hipStreamSynchronize(d->stream));
+    if (!bvh_walk_is_cheaper(*host, kProbeBlocks * 64)) return XT_OK;
     ds.allocs.push_back(own.p);
     ds.bytes += bytes;
     d->used += bytes;

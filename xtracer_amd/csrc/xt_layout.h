@@ -127,13 +127,6 @@ struct XtWideNode {
 #define XT_WIDE_MAX_NODES (1u << 24)
 #define XT_WIDE_LEAF 4u
 #define XT_WIDE_GRID 2047.f
-// Scenes whose primitives fill their boxes worse than this (sum of the boxes'
-// half areas over the primitives' areas) keep the kd-tree walk, whose leaves
-// clip them: a ray meets too many boxes of long thin slanting triangles. Meshes
-// lie at 3.4 (icosphere, terrain: frames in 0.53 to 0.69 of the kd-tree walk's
-// time), the hair strands at 33 (1024x1024, 8 samples: 24.5 ms with the kd-tree
-// walk, 56.2 ms with the BVH).
-#define XT_BVH_MAX_BOX_RATIO 12.0
 
 // Octree node in breadth-first order (children of a node are 8 consecutive
 // nodes). Box rounded outward to FP32. Items are a contiguous range of the

@@ -626,7 +626,7 @@ static __global__ __launch_bounds__(64) void k_bvb_probe(const SceneView S, BvbI
 
     // the walk of k_trace_bvh, one lane a ray
     const f3 inv = mk(rcp_dir(r.d.x), rcp_dir(r.d.y), rcp_dir(r.d.z));
-    const f3 eta = box_slack(r.o, inv, coord_max(S));
+    const f3 eta = box_slack(r.o, inv, slack_base(S));
     const uint32_t oct = octant_of(inv);
     uint32_t grp = 1u << oct, sp = threadIdx.x, nodes = 0, tests = 0;
     while (grp) {

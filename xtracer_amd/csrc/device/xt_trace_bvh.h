@@ -24,6 +24,7 @@
 
 #define XT_W_KEEP 6    // sixteenths of the working lanes at which a phase of a turn ends (3: 3% slower, 8: 1%)
 #define XT_W_FREE 32   // walked rays of a wave at which they are finished for their lanes to help (8: 4% slower at 72 K rays)
+#define XT_W_FAR 1e3f     // scene extents up to which a ray's origin widens the boxes
 #define XT_W_WAVES 4   // waves per SIMD: as many as the LDS of 10 KB a wave leaves room for
 
 // Gathers records of PARTS 16-byte parts into LDS: record `rec` (an index) of
@@ -121,17 +122,34 @@ __device__ __forceinline__ uint32_t octant_order(uint32_t ih, uint32_t oct) {
     return (oct & 4u) ? ((ih << 4) & 0xf0u) | (ih >> 4) : ih;
 }
 
-// Sign bits of a direction, and by how much the walk widens boxes for it.
+// Sign bits of a direction, and by how much the walk widens boxes for it: in
+// proportion to the coordinates, as FP32's misplacement is, but for origins
+// within XT_W_FAR extents of the scene at most. From 1e6 extents away the slack
+// would be the whole scene, and each ray would meet every box; FP32 tells no
+// triangles apart from there.
 __device__ __forceinline__ uint32_t octant_of(f3 inv) {
     return (inv.x < 0.f ? 1u : 0u) | (inv.y < 0.f ? 2u : 0u) | (inv.z < 0.f ? 4u : 0u);
 }
-__device__ __forceinline__ float coord_max(const SceneView &S) {
-    return fmaxf(fmaxf(fmaxf(fabsf(S.kb_lo[0]), fabsf(S.kb_hi[0])), fmaxf(fabsf(S.kb_lo[1]), fabsf(S.kb_hi[1]))),
-                 fmaxf(fabsf(S.kb_lo[2]), fabsf(S.kb_hi[2])));
+struct SlackBase {
+    float scene, far;  // largest coordinates of the scene, and of the origins that slack is given for
+};
+__device__ __forceinline__ SlackBase slack_base(const SceneView &S) {
+    float m = 0.f, ext = 0.f;
+    for (int k = 0; k < 3; ++k) {
+        m = fmaxf(m, fmaxf(fabsf(S.kb_lo[k]), fabsf(S.kb_hi[k])));
+        ext = fmaxf(ext, S.kb_hi[k] - S.kb_lo[k]);
+    }
+    return {m, m + XT_W_FAR * ext};
 }
-__device__ __forceinline__ f3 box_slack(f3 o, f3 inv, float smax) {
-    const float e = XT_W_SLACK * (fmaxf(fabsf(o.x), fmaxf(fabsf(o.y), fabsf(o.z))) + smax);
+__device__ __forceinline__ f3 box_slack(f3 o, f3 inv, SlackBase b) {
+    const float e = XT_W_SLACK * (fminf(fmaxf(fabsf(o.x), fmaxf(fabsf(o.y), fabsf(o.z))), b.far) + b.scene);
     return mk(e * fabsf(inv.x), e * fabsf(inv.y), e * fabsf(inv.z));
+}
+
+// Whether a ray can meet a primitive: one of no direction, or with a NaN or an
+// infinity, passes the tests of boxes and none of a primitive.
+__device__ __forceinline__ bool can_hit(f3 o, f3 d, float dk) {
+    return dk != 0.f && (o.x - o.x) + (o.y - o.y) + (o.z - o.z) + (d.x - d.x) + (d.y - d.y) + (d.z - d.z) == 0.f;
 }
 
 // STACK: the deepest a walk's stack gets, which the tree's depth bounds. A
@@ -156,7 +174,7 @@ static __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(XT_W_
     RaySource R;
     source_init(R, n, waves, T);
     bool more = true;
-    const float smax = coord_max(S);
+    const SlackBase slack = slack_base(S);
 
     bool alive = false, done = false;
     uint32_t ri = 0, origin = XT_NONE, oct = 0, kz = 0;
@@ -251,15 +269,14 @@ static __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(XT_W_
                                 plane32(r.o, r.d, tsmall, S.planes[k], XT_PLANE_BASE + k, best);
                         const float dk = ray_shear(r.d, kz, sx, sy, sz);
                         inv = mk(rcp_dir(r.d.x), rcp_dir(r.d.y), rcp_dir(r.d.z));
-                        eta = box_slack(o, inv, smax);
+                        eta = box_slack(o, inv, slack);
                         oct = octant_of(inv);
                         // the root as the only hit of a group above it
                         grp = 1u << oct;
                         lhit = tn = 0;
                         sp = 0;
                         shared_t = INFINITY;
-                        // a ray of no direction meets no triangle and no sphere
-                        alive = dk != 0.f;
+                        alive = can_hit(o, r.d, dk);
                         done = !alive;
                     }
                 }

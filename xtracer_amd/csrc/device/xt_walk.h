@@ -129,7 +129,9 @@ __device__ __forceinline__ void finish_ray(const SceneView &S, const Queue &in, 
     hit[ri] = make_float4(ht, __uint_as_float(best.prim), hu, hv);
 }
 
-// 1 / x within 1 ulp, +-1e30 near 0
+// 1 / x within 1 ulp, +-1e30 near 0. It places boxes and planes alone: an ulp is
+// a sixteenth of the boxes' slack (XT_W_SLACK) and of the kd walk's widening
+// (XT_KD_EPS), and moves no hit.
 __device__ __forceinline__ float rcp_dir(float x) {
     return fabsf(x) > 1e-30f ? __builtin_amdgcn_rcpf(x) : copysignf(1e30f, x);
 }
@@ -163,11 +165,12 @@ __device__ __forceinline__ float tri_box_entry(f3 A, f3 B, f3 C, f3 inv, f3 eta)
 }
 
 // tri32 and offer() in one straight line: the tests' rare outcomes (a
-// deferral) share one branch. Same decisions, in the same order; but with BOX a
-// grazed triangle is deferred from where the ray enters its box (rinv, eta: the
-// ray's reciprocal direction and the slack of the walk's boxes) and not from the ray's origin: a walk that visits
-// the tree in another order, and so tests other triangles behind the closest
-// hit, decides alike which rays are re-checked.
+// deferral) share one branch. The same values, rounded alike, and the same
+// decisions; but with BOX a grazed triangle is deferred from where the ray
+// enters its box (rinv, eta: the ray's reciprocal direction and the slack of the
+// walk's boxes) and not from the ray's origin: a walk that visits the tree in
+// another order, and so tests other triangles behind the closest hit, decides
+// alike which rays are re-checked.
 template <bool BOX>
 __device__ __forceinline__ void tri32_flat(const f3 o, float sx, float sy, float sz, uint32_t kz, const float4 a,
                                            const float4 b, const float4 c, uint32_t prim, Best &best, f3 rinv,
@@ -182,7 +185,7 @@ __device__ __forceinline__ void tri32_flat(const f3 o, float sx, float sy, float
     const float cx = (k0 ? C.y : (k1 ? C.z : C.x)) - sx * cz, cy = (k0 ? C.z : (k1 ? C.x : C.y)) - sy * cz;
     const float U = edge2(cx, by, cy, bx), V = edge2(ax, cy, ay, cx), W = edge2(bx, ay, by, ax);
     const float det = U + V + W;
-    const float inv = __builtin_amdgcn_rcpf(det);
+    const float inv = 1.f / det;
     const float t = (U * az + V * bz + W * cz) * sz * inv;
     const float m = fminf(fminf(V * inv, W * inv), U * inv);
     const bool live = !(XT_PRIM_FLAGS(tf) & XT_PF_DEGENERATE);

@@ -248,7 +248,7 @@ typedef struct xt_tuning {
                                  its pixels cut into that many groups whose rounds run on streams of their
                                  own, so that one group's shading and launch tails overlap another's trace;
                                  images are the same bits either way; 2 leaves passes below 2^19 paths
-                                 in one group (2) */
+                                 in one group, but for octree jobs on 1024 primitives or more (2) */
 } xt_tuning;
 int xt_dev_set_tuning(xt_dev *d, const xt_tuning *t);
 int xt_dev_get_tuning(const xt_dev *d, xt_tuning *t);

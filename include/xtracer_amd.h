@@ -276,8 +276,9 @@ int xt_trace(xt_dev *d, uint32_t scene_id, int accel, const xt_rays *rays, xt_hi
  * ray1[i] = (dx, dy, dz, 0) as float4, where `origin` holds the bits of the
  * primitive id the ray leaves from (XT_HIT_NONE for a free ray); hit[i] =
  * (t, prim bits, u, v) as float4.
- * Runs on the device's stream; *kernel_ms (optional) gets the trace kernel
- * time measured with HIP events on that stream. */
+ * Runs on the device's stream; *kernel_ms (optional) gets the trace kernel's
+ * time by the device's wall clock: from the start of its first workgroup to
+ * the start of the kernel behind it. */
 int xt_trace_device(xt_dev *d, uint32_t scene_id, int accel, const void *ray0, const void *ray1, void *hit,
                     uint32_t *flags, uint64_t n, float *kernel_ms);
 
@@ -316,7 +317,7 @@ typedef struct xt_job_stats {
     uint64_t retests;      /* rays re-tested in FP64 */
     uint64_t samples;      /* camera samples */
     double ms_total;       /* device time of the render, HIP events */
-    double ms_trace;       /* sum of trace kernel times */
+    double ms_trace;       /* sum of trace kernel times (as xt_trace_device's, up to 256 launches) */
     uint32_t trace_launches;
     uint32_t passes;
     double latency_ms;     /* serving: completion - submission */

@@ -552,7 +552,7 @@ __device__ __forceinline__ uint32_t object_of(const SceneView &S, uint32_t p) {
 // the full re-test, as do the rays listed for it: the FP64 walk. ray64
 // (optional) holds the FP64 rays by path id; otherwise the FP32 ray is widened.
 // One launch for both lists: usually few rays or none (1 in 13,000 of the 1080p
-// icosphere frame is re-checked, 3 of 78 M re-tested), and a launch costs about
+// icosphere frame is re-checked, 2 of 72 M re-tested), and a launch costs about
 // 4 us. Bound by the longest FP64 walk. One-wave blocks: the 50 KB of stacks of
 // a four-wave block wait for a compute unit that a trace of another group has
 // left (hair strands frame 24.4 ms, with one-wave blocks 23.6).

@@ -14,7 +14,10 @@
 // frame 236 to 191, 256x256x4 paths 715 to 560, and the end of larger launches
 // (4 M random rays 710 to 545, 1080p 16 spp paths 16.2 to 15.0 ms).
 //
-// Bound by VALU issue (80% of the time on the 1080p icosphere frame). What it
+// Bound by VALU issue and by the return of its gathers: on the 1080p icosphere
+// frame the vector units are busy 71% of the time, at 38 of 64 lanes, and the
+// texture data units 81%, three quarters of that waiting for L1 and L2; on 4 M
+// random rays 63% at 31 lanes, and 84%. What it
 // measured, trace time of that frame's 72.1 M queries with the launches one
 // after another: kd-tree walk 15.5 ms, this 9.4 ms; 4 M random rays 1256 to
 // 718 us. With 80-byte nodes of 8-bit planes (48 conversions more per node)
@@ -131,7 +134,7 @@ __device__ __forceinline__ uint32_t octant_of(f3 inv) {
     return (inv.x < 0.f ? 1u : 0u) | (inv.y < 0.f ? 2u : 0u) | (inv.z < 0.f ? 4u : 0u);
 }
 struct SlackBase {
-    float scene, far;  // largest coordinates of the scene, and of the origins that slack is given for
+    float scene, far;  // slack of the scene's coordinates; the largest coordinate of an origin that slack is given for
 };
 __device__ __forceinline__ SlackBase slack_base(const SceneView &S) {
     float m = 0.f, ext = 0.f;
@@ -139,17 +142,17 @@ __device__ __forceinline__ SlackBase slack_base(const SceneView &S) {
         m = fmaxf(m, fmaxf(fabsf(S.kb_lo[k]), fabsf(S.kb_hi[k])));
         ext = fmaxf(ext, S.kb_hi[k] - S.kb_lo[k]);
     }
-    return {m, m + XT_W_FAR * ext};
+    return {XT_W_SLACK * m, m + XT_W_FAR * ext};
 }
 __device__ __forceinline__ f3 box_slack(f3 o, f3 inv, SlackBase b) {
-    const float e = XT_W_SLACK * (fminf(fmaxf(fabsf(o.x), fmaxf(fabsf(o.y), fabsf(o.z))), b.far) + b.scene);
+    const float e = XT_W_SLACK * fminf(fmaxf(fabsf(o.x), fmaxf(fabsf(o.y), fabsf(o.z))), b.far) + b.scene;
     return mk(e * fabsf(inv.x), e * fabsf(inv.y), e * fabsf(inv.z));
 }
 
 // Whether a ray can meet a primitive: one of no direction, or with a NaN or an
 // infinity, passes the tests of boxes and none of a primitive.
 __device__ __forceinline__ bool can_hit(f3 o, f3 d, float dk) {
-    return dk != 0.f && (o.x - o.x) + (o.y - o.y) + (o.z - o.z) + (d.x - d.x) + (d.y - d.y) + (d.z - d.z) == 0.f;
+    return dk != 0.f && fabsf(o.x) + fabsf(o.y) + fabsf(o.z) + fabsf(d.x) + fabsf(d.y) + fabsf(d.z) < INFINITY;
 }
 
 // STACK: the deepest a walk's stack gets, which the tree's depth bounds. A

@@ -120,5 +120,5 @@ class XtScratch {
 };
 
 // The first block of a scene's index builds: the kd-tree build of the terrain
-// holds 420 bytes a primitive at its largest level, a wide BVH build 400.
+// holds 420 bytes a primitive at its largest level, a wide BVH build 364.
 inline size_t xt_build_block(uint32_t n_prims) { return 512ull * n_prims + (1u << 21); }

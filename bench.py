@@ -32,8 +32,16 @@ TRACE_BYTES_PER_QUERY = 48      # read ray (2 x float4) + write hit (float4)
 PIPE_BYTES_PER_QUERY = 184      # ray/hit/path-state streams of trace + shade + compaction
 PIPE_BYTES_PER_SAMPLE = 152     # camera ray + state write, FP64 accumulate read + write
 TRACE_KERNEL = "k_trace"
+
 COPY_KERNEL = "__amd_rocclr_copyBuffer"
 COPY_PROBE_MIB = 1024
+
+
+def trace_kernel(dev, sid, accel):
+    """The trace kernel that walks the scene."""
+    if accel == "octree":
+        return "k_trace_oct (octree)"
+    return "k_trace_bvh (wide BVH)" if dev.index_stats(sid)["bvh_depth"] else "k_trace_kd (kd-tree)"
 
 
 def log(msg):
@@ -550,7 +558,7 @@ def main():
                      "traffic_per_query": probe.get("bytes_per_query") if probe else None,
                      "l2_hit_rate": probe.get("l2_hit_rate") if probe else None,
                      "traffic_probe": probe,
-                     "kernel": "k_trace_bvh (wide BVH)", "bytes_per_query": TRACE_BYTES_PER_QUERY,
+                     "kernel": trace_kernel(dev, sid, args.accel), "bytes_per_query": TRACE_BYTES_PER_QUERY,
                      "avg_launch_ms": round(trace_ms / max(1, launches), 4), "launches": launches,
                      "busy_ms_per_frame": round(busy_ms / max(1, args.steps), 3),
                      "concurrent_groups": tuning.get("frame_lanes", 1),

@@ -445,6 +445,12 @@ class Device:
         self._check(lib().xt_scene_build_kd_device(self._d, scene_id, ctypes.byref(p), ctypes.byref(st)))
         return st.as_dict()
 
+    def index_stats(self, scene_id):
+        """The resident trees' sizes and depths, without the trees."""
+        st = KdBuildStats()
+        self._check(lib().xt_scene_get_kd_device(self._d, scene_id, None, None, None, ctypes.byref(st)))
+        return st.as_dict()
+
     def kdtree(self, scene_id):
         """The resident kd-tree: nodes (n, 2) uint32, refs, bounds (6,), stats."""
         st = KdBuildStats()

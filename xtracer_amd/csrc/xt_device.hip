@@ -459,61 +459,38 @@ int xt_scene_release(xt_dev *d, uint32_t scene_id) {
 
 }  // extern "C"
 
-// Instantiations of the kd-tree trace kernel over the tuning space. The
-// persistent grid is `per_cu` blocks per CU, or (per_cu == 0) exactly the
-// blocks the CU keeps resident, from the occupancy calculator.
-template <int STACK, int BS>
-static void launch_kd_trace_sb(unsigned per_cu, int n_cu, size_t cap, hipStream_t st, const SceneView &v,
-                               const Queue &q, const uint32_t *count, float4 *hit, uint32_t *retest, uint4 *recheck, const TraceCtl &T) {
+typedef void (*TraceKernel)(const SceneView, const Queue, const uint32_t *, float4 *, uint32_t *, uint4 *,
+                            const TraceCtl);
+
+// A persistent trace kernel: `per_cu` blocks per CU, or (per_cu == 0) exactly
+// the blocks the CU keeps resident, from the occupancy calculator.
+template <TraceKernel K, int BS>
+static void launch_resident(unsigned per_cu, int n_cu, size_t cap, hipStream_t st, const SceneView &v, const Queue &q,
+                            const uint32_t *count, float4 *hit, uint32_t *retest, uint4 *recheck, const TraceCtl &T) {
     static int resident = 0;
     if (per_cu == 0) {
         if (resident == 0) {
             int nb = 0;
-            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_trace_kd<STACK, BS>, BS, 0) !=
-                    hipSuccess ||
-                nb < 1)
-                nb = 1;
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, K, BS, 0) != hipSuccess || nb < 1) nb = 1;
             resident = nb;
         }
         per_cu = (unsigned)resident;
     }
     const size_t need = (cap + BS / 64 - 1) / (BS / 64);  // a wave for every ray
     const unsigned g = (unsigned)std::max<size_t>(1, std::min<size_t>(need, (size_t)n_cu * per_cu));
-    hipLaunchKernelGGL((k_trace_kd<STACK, BS>), dim3(g), dim3(BS), 0, st, v, q, count, hit, retest, recheck, T);
+    hipLaunchKernelGGL(K, dim3(g), dim3(BS), 0, st, v, q, count, hit, retest, recheck, T);
 }
 
-template <int STACK, int BS>
-static void launch_bvh_trace_sb(unsigned per_cu, int n_cu, size_t cap, hipStream_t st, const SceneView &v,
-                                const Queue &q, const uint32_t *count, float4 *hit, uint32_t *retest, uint4 *recheck,
-                                const TraceCtl &T) {
-    static int resident = 0;
-    if (per_cu == 0) {
-        if (resident == 0) {
-            int nb = 0;
-            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_trace_bvh<STACK, BS>, BS, 0) != hipSuccess || nb < 1)
-                nb = 1;
-            resident = nb;
-        }
-        per_cu = (unsigned)resident;
-    }
-    const size_t need = (cap + BS / 64 - 1) / (BS / 64);  // a wave for every ray
-    const unsigned g = (unsigned)std::max<size_t>(1, std::min<size_t>(need, (size_t)n_cu * per_cu));
-    hipLaunchKernelGGL((k_trace_bvh<STACK, BS>), dim3(g), dim3(BS), 0, st, v, q, count, hit, retest, recheck, T);
+// The instances over the tuning space.
+template <int STACK, class... A>
+static void launch_bvh_trace_s(unsigned bs, const A &...a) {
+    if (bs == 128) launch_resident<k_trace_bvh<STACK, 128>, 128>(a...);
+    else launch_resident<k_trace_bvh<STACK, 256>, 256>(a...);
 }
-
-template <int STACK>
-static void launch_bvh_trace_s(unsigned bs, unsigned per_cu, int n_cu, size_t cap, hipStream_t st, const SceneView &v,
-                               const Queue &q, const uint32_t *count, float4 *hit, uint32_t *retest, uint4 *recheck,
-                               const TraceCtl &T) {
-    if (bs == 128) launch_bvh_trace_sb<STACK, 128>(per_cu, n_cu, cap, st, v, q, count, hit, retest, recheck, T);
-    else launch_bvh_trace_sb<STACK, 256>(per_cu, n_cu, cap, st, v, q, count, hit, retest, recheck, T);
-}
-
-template <int STACK>
-static void launch_kd_trace_s(unsigned bs, unsigned per_cu, int n_cu, size_t cap, hipStream_t st, const SceneView &v,
-                              const Queue &q, const uint32_t *count, float4 *hit, uint32_t *retest, uint4 *recheck, const TraceCtl &T) {
-    if (bs == 128) launch_kd_trace_sb<STACK, 128>(per_cu, n_cu, cap, st, v, q, count, hit, retest, recheck, T);
-    else launch_kd_trace_sb<STACK, 256>(per_cu, n_cu, cap, st, v, q, count, hit, retest, recheck, T);
+template <int STACK, class... A>
+static void launch_kd_trace_s(unsigned bs, const A &...a) {
+    if (bs == 128) launch_resident<k_trace_kd<STACK, 128>, 128>(a...);
+    else launch_resident<k_trace_kd<STACK, 256>, 256>(a...);
 }
 
 static void launch_kd_trace(const xt_tuning &tn, uint32_t bvh_depth, int n_cu, size_t cap, hipStream_t st, const SceneView &view,
@@ -526,7 +503,7 @@ static void launch_kd_trace(const xt_tuning &tn, uint32_t bvh_depth, int n_cu, s
         const uint32_t s = bvh_depth < 2 ? 0 : bvh_depth - 2;
         if (s <= 8) launch_bvh_trace_s<8>(bs, pc, n_cu, cap, st, v, q, count, hit, retest, recheck, T);
         else if (s <= 12) launch_bvh_trace_s<12>(bs, pc, n_cu, cap, st, v, q, count, hit, retest, recheck, T);
-        else launch_bvh_trace_sb<24, 128>(pc, n_cu, cap, st, v, q, count, hit, retest, recheck, T);
+        else launch_resident<k_trace_bvh<24, 128>, 128>(pc, n_cu, cap, st, v, q, count, hit, retest, recheck, T);
         return;
     }
     switch (tn.kd_stack) {

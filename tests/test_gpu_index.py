@@ -136,6 +136,20 @@ def test_equal_primitives_walk_the_bvh(device, tmp_path):
 
 
 @pytest.mark.gpu
+def test_boxes_beyond_the_builds_range_stay_on_the_kd_tree(device, tmp_path):
+    """One triangle at 1e30 among ordinary ones: its box's area is not finite."""
+    rng = np.random.default_rng(4)
+    tris = rng.uniform(-2, 2, (300, 1, 3)) + rng.normal(scale=0.05, size=(300, 3, 3))
+    s = _soup(tmp_path, np.concatenate([tris, 1e30 * (1.0 + np.eye(3)[None])]))
+    assert _depth(device, s) == 0
+    o = rng.normal(size=(2000, 3))
+    o *= (9.0 / np.linalg.norm(o, axis=1))[:, None]
+    d = tris.mean(axis=1)[rng.integers(300, size=2000)] - o
+    d /= np.linalg.norm(d, axis=1)[:, None]
+    _check(device, s, o, d)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("kind,kw,bvh", [("spheres", {}, True), ("icosphere", {"subdiv": 5}, True),
                                          ("terrain", {"n": 41}, True), ("strands", {"strands": 600}, True),
                                          ("strands", {"strands": 600, "step": 0.4}, False)])
